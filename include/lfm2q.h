@@ -162,6 +162,24 @@ int lfm2q_gemv_chain_noalloc(const lfm2q_gemv_op *ops, const lfm2q_gemv_op *ops_
  * Replaces launch_silu_mul kernels/lfm2_decode.cu:954-969 (bound as silu_mul(), kernels/lfm2_decode.cpp:100-103). */
 int lfm2q_silu_mul(const lfm2q_bf16 *g, lfm2q_bf16 *y, int B, int I, lfm2q_stream_t stream);
 
+/* ------------------------------------------------------------------------------------------ decode step ops */
+
+/* One decode step's attention of one layer, at position ctr[0] (read on the device) of a static cache: every q head
+ * and k head of qkv bf16 [B, (n_heads + 2 n_kv) head_dim] RMS-normalized and rotated, the new key and value written into
+ * the cache at that position, out bf16 [B, n_heads head_dim] = softmax(scale q k^T) v over positions 0 .. ctr[0], all in
+ * fp32 from the bf16 operands (the new key rounded to bf16 first, as later steps read it).
+ * qk_w fp32 [2, n_heads + n_kv, head_dim]: the head weights w (q heads, then k heads), then (-w[half:], w[:half]); rope
+ * fp32 [max_len, 2, head_dim]: cos and sin per position; k bf16 [B, n_kv, head_dim, max_len] (keys transposed), v bf16
+ * [B, n_kv, max_len, head_dim]. head_dim 64, n_heads / n_kv in {1, 2, 4, 8}, max_len % 8 == 0; qkv, k, v 16-byte
+ * aligned. ws: lfm2q_attn_step_workspace_bytes() of device memory (may be 0), contents irrelevant, not shared by
+ * overlapping calls. A position outside the cache is a device trap.
+ * Replaces the reference step's q / k norm, rotary embedding, cache write and attention (src/lfm2opt/runtime.py:
+ * 256-271). */
+int lfm2q_attn_step(const lfm2q_bf16 *qkv, const float *qk_w, const float *rope, const int64_t *ctr, lfm2q_bf16 *k,
+                    lfm2q_bf16 *v, lfm2q_bf16 *out, int B, int n_heads, int n_kv, int head_dim, int max_len, float scale,
+                    float eps, void *ws, size_t ws_bytes, lfm2q_stream_t stream);
+size_t lfm2q_attn_step_workspace_bytes(int B, int n_heads, int n_kv, int max_len);
+
 /* ------------------------------------------------------------------------------------------ W8A8 GEMM */
 
 /* Per-token activation quantization: s[r] = max(max_k |x[r, k]|, 1e-8) / 127 (IEEE division),

@@ -24,7 +24,8 @@ class GemvOp(ctypes.Structure):
 
 
 # entry points that return something other than an int status
-RESTYPES = {"lfm2q_gemv_chain_workspace_bytes": ctypes.c_size_t, "lfm2q_gemm_workspace_bytes": ctypes.c_size_t}
+RESTYPES = {"lfm2q_gemv_chain_workspace_bytes": ctypes.c_size_t, "lfm2q_gemm_workspace_bytes": ctypes.c_size_t,
+            "lfm2q_attn_step_workspace_bytes": ctypes.c_size_t}
 
 # name -> argument types (every entry point returns an int status unless listed in RESTYPES)
 SIGNATURES = {
@@ -34,6 +35,8 @@ SIGNATURES = {
     "lfm2q_gemv_residual": [_I, _P, _P, _P, _P, _I, _I, _I, _P],
     "lfm2q_gemv_rmsnorm": [_I, _I, _P, _P, _P, _P, _F, _P, _I, _I, _P],
     "lfm2q_gemv_w4": [_I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
+    "lfm2q_attn_step": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _P, ctypes.c_size_t, _P],
+    "lfm2q_attn_step_workspace_bytes": [_I, _I, _I, _I],
     "lfm2q_silu_mul": [_P, _P, _I, _I, _P],
     "lfm2q_quant_rows": [_P, _P, _P, _I, _I, _P],
     "lfm2q_quant_groups": [_P, _P, _P, _I, _I, _P],

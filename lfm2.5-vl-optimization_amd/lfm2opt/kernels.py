@@ -208,6 +208,35 @@ class DecodeOps:
         _capi.call("lfm2q_gemv_residual", wtype, W.data_ptr(), _capi.ptr(scale), x.data_ptr(), h.data_ptr(), B, N,
                    K, _capi.stream(x))
 
+    @staticmethod
+    def attn_step_workspace(B, n_heads, n_kv, max_len, device):
+        """The workspace attn_step needs for this shape (fp32; may be empty). Calls that share one must not overlap."""
+        n = _capi.lib().lfm2q_attn_step_workspace_bytes(B, n_heads, n_kv, max_len)
+        return torch.empty(n // 4, dtype=torch.float32, device=device)
+
+    def attn_step(self, qkv, qk_w, rope, ctr, k, v, out, scale, eps, ws):
+        """One decode step's attention of one layer (an addition): q / k head RMSNorm and rotary embedding of qkv
+        [B, (nh + 2 nkv) 64], the new key and value into k [B, nkv, 64, max_len] / v [B, nkv, max_len, 64] at position
+        ctr[0], out [B, nh 64] = attention over positions 0 .. ctr[0]. qk_w fp32 [2, nh + nkv, 64], rope fp32 [max_len,
+        2, 64], ctr int64 (lfm2q_attn_step). Replaces the step's attention ops, src/lfm2opt/runtime.py:256-271."""
+        for t, name in ((qkv, "qkv"), (k, "k"), (v, "v"), (out, "out")):
+            _check_bf16(t, name)
+        for t, dt, name in ((qk_w, torch.float32, "qk_w"), (rope, torch.float32, "rope"), (ctr, torch.int64, "ctr"),
+                            (ws, torch.float32, "ws")):
+            _check_t(t, dt, name)
+        if not (k.dim() == 4 and v.dim() == 4 and qk_w.dim() == 3):
+            raise RuntimeError("attn_step: k [B, nkv, hd, max_len], v [B, nkv, max_len, hd], qk_w [2, nh + nkv, hd]")
+        B, nkv, hd, max_len = k.shape
+        nh = qk_w.size(1) - nkv
+        if not (tuple(v.shape) == (B, nkv, max_len, hd) and qk_w.size(0) == 2 and qk_w.size(2) == hd and nh >= 1
+                and qkv.numel() == B * (nh + 2 * nkv) * hd and out.numel() == B * nh * hd
+                and rope.numel() >= max_len * 2 * hd and ctr.numel() >= 1):
+            raise RuntimeError("attn_step: shapes")
+        _same_device(qkv, qk_w, rope, ctr, k, v, out, ws)
+        _capi.call("lfm2q_attn_step", qkv.data_ptr(), qk_w.data_ptr(), rope.data_ptr(), ctr.data_ptr(), k.data_ptr(),
+                   v.data_ptr(), out.data_ptr(), B, nh, nkv, hd, max_len, float(scale), float(eps), ws.data_ptr(),
+                   ws.numel() * 4, _capi.stream(qkv))
+
     def _epi_args(self, W, scale, x, y, rows_per_out):
         _check_bf16(x, "x")
         _check_bf16(y, "y")

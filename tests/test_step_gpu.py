@@ -1,0 +1,82 @@
+"""The decode step's non-matmul kernels (csrc/step.hip) against fp64 on the CPU, at the sizes where they can go wrong:
+the edges of a chunk of 256 positions, of a 16-byte run of positions and of the splits, every head grouping."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# attn_step: the output is one bf16 rounding (2^-9 of the value) of fp32 sums over at most 4,096 positions of values up
+# to max |v|; q stays fp32, so its own error is the exp2 of an fp32 score (|score| < 2^6: 2^-18). 2^-8 of the largest
+# value covers all of it.
+ATTN_TOL = 2.0 ** -8
+
+
+def attention_reference(qkv, qk_w, rope, pos, k, v, scale, eps):
+    """fp64: (out, the new key, the new value); k [B, nkv, 64, max_len], v [B, nkv, max_len, 64]."""
+    B, nkv, hd, _ = k.shape
+    nh = qk_w.shape[1] - nkv
+    x = qkv.double().view(B, nh + 2 * nkv, hd)
+    qk = x[:, :nh + nkv]
+    n = qk * torch.rsqrt(qk.pow(2).mean(-1, keepdim=True) + eps) * qk_w[0].double()
+    cos, sin = rope[pos].double()
+    rot = torch.cat((-n[..., hd // 2:], n[..., :hd // 2]), -1)
+    r = n * cos + rot * sin
+    q, kn, vn = r[:, :nh], r[:, nh:].to(torch.bfloat16), x[:, nh + nkv:]
+    ks = torch.cat((k[..., :pos].double(), kn.double()[..., None]), -1)
+    vs = torch.cat((v[:, :, :pos].double(), vn[:, :, None]), 2)
+    p = torch.softmax(torch.matmul(q.view(B, nkv, nh // nkv, hd), ks) * scale, -1)
+    return torch.matmul(p, vs).reshape(B, nh * hd), kn, vn.to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+@pytest.mark.parametrize("B,max_len,positions", [(1, 8, (0, 3, 7)), (2, 256, (0, 31, 255)), (1, 264, (256, 263)),
+                                                 (3, 512, (255, 256, 511)), (1, 1032, (767, 768, 1031)),
+                                                 (1, 4096, (2047, 4095)), (40, 1280, (0, 300, 1279))])
+def test_attn_step(cuda, G, B, max_len, positions):
+    from lfm2opt.kernels import ext
+
+    E, nkv, hd, eps, scale = ext(), 2, 64, 1e-5, 64 ** -0.5
+    nh = G * nkv
+    for pos in positions:
+        print(f"attn_step G={G} B={B} max_len={max_len} pos={pos}", flush=True)
+        g = torch.Generator().manual_seed(pos + G)
+        qkv = torch.randn(B, (nh + 2 * nkv) * hd, generator=g).to(torch.bfloat16)
+        w = 1 + 0.2 * torch.randn(nh + nkv, hd, generator=g)
+        qk_w = torch.stack((w, torch.cat((-w[:, hd // 2:], w[:, :hd // 2]), -1)))
+        ang = torch.rand(max_len, hd // 2, generator=g).repeat(1, 2) * 6
+        rope = torch.stack((ang.cos(), ang.sin()), 1)
+        k = (torch.randn(B, nkv, hd, max_len, generator=g) * 2).to(torch.bfloat16)
+        v = torch.randn(B, nkv, max_len, hd, generator=g).to(torch.bfloat16)
+        k[..., pos:] = float("nan")  # unwritten slots are never read
+        v[:, :, pos:] = float("nan")
+        want, kn, vn = attention_reference(qkv, qk_w, rope, pos, k, v, scale, eps)
+        kd, vd = k.to(cuda), v.to(cuda)
+        out = torch.empty(B, nh * hd, device=cuda, dtype=torch.bfloat16)
+        ctr = torch.tensor([pos, 0], device=cuda)
+        E.attn_step(qkv.to(cuda), qk_w.to(cuda), rope.to(cuda), ctr, kd, vd, out, scale, eps,
+                    E.attn_step_workspace(B, nh, nkv, max_len, cuda))
+        err = (out.cpu().double() - want).abs().max()
+        assert err <= ATTN_TOL * max(1.0, float(want.abs().max())), f"pos {pos}: {err:.3e}"
+        kc, vc = kd.cpu(), vd.cpu()
+        assert torch.equal(vc[:, :, pos], vn)
+        assert (kc[..., pos].double() - kn.double()).abs().max() <= 2.0 ** -8 * float(kn.double().abs().max())
+        assert torch.equal(kc[..., :pos], k[..., :pos]) and torch.equal(vc[:, :, :pos], v[:, :, :pos])
+        assert kc[..., pos + 1:].isnan().all() and vc[:, :, pos + 1:].isnan().all()
+
+
+def test_attn_step_refuses_other_shapes(cuda):
+    from lfm2opt.kernels import ext
+
+    E, bf = ext(), torch.bfloat16
+
+    def call(nh, nkv, hd, max_len):
+        z = lambda *s, dt=bf: torch.zeros(*s, dtype=dt, device=cuda)  # noqa: E731
+        E.attn_step(z(1, (nh + 2 * nkv) * hd), z(2, nh + nkv, hd, dt=torch.float32),
+                    z(max_len, 2, hd, dt=torch.float32), z(2, dt=torch.int64), z(1, nkv, hd, max_len),
+                    z(1, nkv, max_len, hd), z(1, nh * hd), 0.1, 1e-5, z(0, dt=torch.float32))
+
+    for args, what in (((4, 2, 32, 64), "head_dim"), ((6, 2, 64, 64), "1, 2, 4 or 8"), ((4, 2, 64, 12), "multiple of 8"),
+                       ((4, 2, 64, 4096), "workspace")):
+        with pytest.raises(RuntimeError, match=what):
+            call(*args)
