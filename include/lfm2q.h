@@ -180,6 +180,15 @@ int lfm2q_attn_step(const lfm2q_bf16 *qkv, const float *qk_w, const float *rope,
                     float eps, void *ws, size_t ws_bytes, lfm2q_stream_t stream);
 size_t lfm2q_attn_step_workspace_bytes(int B, int n_heads, int n_kv, int max_len);
 
+/* One decode step of a gated short convolution at position ctr[0] (read on the device): of bcx bf16 [B, 3 H] = b | c | x,
+ * b x goes to row ctr[0] mod L of ring bf16 [L, B, H] (the last L positions' b x), and out bf16 [B, H] = c (sum over
+ * the ring of each position's value times its tap + bias), with the roundings of the bf16 tensor ops: b x, each tap's
+ * product, their fp32 sum, the biased sum, the gated output. wt bf16 [L, H]: tap L - 1 multiplies the newest position;
+ * bias bf16 [H] or NULL. H % 4 == 0, 1 <= L <= 8, 8-byte aligned tensors.
+ * Replaces the short-conv step of gemv_epi(1, ...) kernels/lfm2_decode.cu:724-805 without its projection. */
+int lfm2q_conv_step(const lfm2q_bf16 *bcx, lfm2q_bf16 *ring, const lfm2q_bf16 *wt, const lfm2q_bf16 *bias,
+                    const int64_t *ctr, lfm2q_bf16 *out, int B, int H, int L, lfm2q_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------ W8A8 GEMM */
 
 /* Per-token activation quantization: s[r] = max(max_k |x[r, k]|, 1e-8) / 127 (IEEE division),

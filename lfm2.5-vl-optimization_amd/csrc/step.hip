@@ -1,5 +1,6 @@
 // The non-matmul ops of one LFM2 decode step on gfx950, each as one or two launches over the runtime's static buffers:
 //   attn_step   q / k head RMSNorm and rotary embedding, the new key and value into the cache, attention over it
+//   conv_step   the gated short convolution: B x into its ring of the last inputs, the newest output, the gate C
 //
 // Reference: the decode step's fused ops of src/lfm2opt/runtime.py:246-294 (its CUDA kernels of kernels/lfm2_decode.cu).
 #include "common.hpp"
@@ -274,6 +275,62 @@ inline AttnShape attn_shape(int B, int nkv, int grp, int max_len) {
     return {chunks, splits, heads};
 }
 
+// ------------------------------------------------------------------------------------------------ short convolution
+// Thread: 4 channels of one batch row. ring [L, B, H] holds B x of the last L positions, position p in row p mod L; at
+// position p ring row s holds p - (p - s) mod L, which tap L - 1 - (p - s) mod L multiplies (wt [L, H]). Rounded as
+// transformers' bf16 step: B x, each tap's product, their fp32 sum (in ring order), with the bias, and times C. Latency:
+// a few loads deep, so few channels per thread and many workgroups. The three-layer INT4 step lost 23 us with it, two
+// layers of six PyTorch launches (~14 us of kernels each) against two of this one (~2 us).
+constexpr int CONV_MAX = 8;  // longest ring
+
+template <int L>
+__global__ __launch_bounds__(64) void conv_step_kernel(const uint16_t *__restrict__ bcx, uint16_t *__restrict__ ring,
+                                                       const uint16_t *__restrict__ wt,
+                                                       const uint16_t *__restrict__ bias,
+                                                       const int64_t *__restrict__ ctr, uint16_t *__restrict__ out,
+                                                       int B, int H) {
+#pragma clang fp contract(off)
+    const int c = 4 * (blockIdx.x * 64 + threadIdx.x), b = blockIdx.y;
+    if (c >= H) return;
+    const uint16_t *row = bcx + (size_t)b * 3 * H + c;
+    const uint2 vb = *reinterpret_cast<const uint2 *>(row), vc = *reinterpret_cast<const uint2 *>(row + H),
+                vx = *reinterpret_cast<const uint2 *>(row + 2 * H);
+    uint2 rv[L], wv[L];
+#pragma unroll
+    for (int s = 0; s < L; ++s) {
+        rv[s] = *reinterpret_cast<const uint2 *>(ring + ((size_t)s * B + b) * H + c);
+        wv[s] = *reinterpret_cast<const uint2 *>(wt + (size_t)s * H + c);
+    }
+    const uint2 bv = bias ? *reinterpret_cast<const uint2 *>(bias + c) : make_uint2(0, 0);
+    const int r = (int)((ctr[0] % L + L) % L);
+    const uint2 u = make_uint2(pack_bf16x2(bf2f_lo(vb.x) * bf2f_lo(vx.x), bf2f_hi(vb.x) * bf2f_hi(vx.x)),
+                               pack_bf16x2(bf2f_lo(vb.y) * bf2f_lo(vx.y), bf2f_hi(vb.y) * bf2f_hi(vx.y)));
+    *reinterpret_cast<uint2 *>(ring + ((size_t)r * B + b) * H + c) = u;
+    float y[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < L; ++s) {
+        const uint2 v = s == r ? u : rv[s];
+        const int tap = s <= r ? L - 1 - (r - s) : s - r - 1;
+        uint2 w = wv[0];
+#pragma unroll
+        for (int k = 1; k < L; ++k)
+            if (k == tap) w = wv[k];
+        y[0] += rbf(bf2f_lo(v.x) * bf2f_lo(w.x));
+        y[1] += rbf(bf2f_hi(v.x) * bf2f_hi(w.x));
+        y[2] += rbf(bf2f_lo(v.y) * bf2f_lo(w.y));
+        y[3] += rbf(bf2f_hi(v.y) * bf2f_hi(w.y));
+    }
+    const float bf[4] = {bf2f_lo(bv.x), bf2f_hi(bv.x), bf2f_lo(bv.y), bf2f_hi(bv.y)};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        y[e] = rbf(y[e]);
+        if (bias) y[e] = rbf(y[e] + bf[e]);
+    }
+    *reinterpret_cast<uint2 *>(out + (size_t)b * H + c) =
+        make_uint2(pack_bf16x2(bf2f_lo(vc.x) * y[0], bf2f_hi(vc.x) * y[1]),
+                   pack_bf16x2(bf2f_lo(vc.y) * y[2], bf2f_hi(vc.y) * y[3]));
+}
+
 }  // namespace
 }  // namespace lfm2q
 
@@ -322,4 +379,30 @@ extern "C" int lfm2q_attn_step(const lfm2q_bf16 *qkv, const float *qk_w, const f
         attn_combine_kernel<<<(B * n_heads + 3) / 4, 256, 0, st>>>(part, ctr, out, B * n_heads, max_len, s.chunks,
                                                                    s.splits);
     return launch_status("attn_step");
+}
+
+extern "C" int lfm2q_conv_step(const lfm2q_bf16 *bcx, lfm2q_bf16 *ring, const lfm2q_bf16 *wt, const lfm2q_bf16 *bias,
+                               const int64_t *ctr, lfm2q_bf16 *out, int B, int H, int L, lfm2q_stream_t stream) {
+    LFM2Q_REQUIRE(bcx && ring && wt && ctr && out, LFM2Q_ERR_ARG, "conv_step: null pointer");
+    LFM2Q_REQUIRE(B >= 1 && B <= 65535 && H >= 4 && H % 4 == 0, LFM2Q_ERR_SHAPE,
+                  "conv_step: need 1 <= B <= 65535 and H %% 4 == 0 (B=%d H=%d)", B, H);
+    LFM2Q_REQUIRE(((((uintptr_t)bcx | (uintptr_t)ring | (uintptr_t)wt) | ((uintptr_t)bias | (uintptr_t)out)) & 7) == 0,
+                  LFM2Q_ERR_ALIGN, "conv_step: tensors must be 8-byte aligned");
+    const dim3 grid((H / 4 + 63) / 64, B);
+    const hipStream_t st = (hipStream_t)stream;
+#define LFM2Q_CONV(L_) \
+    case L_: conv_step_kernel<L_><<<grid, 64, 0, st>>>(bcx, ring, wt, bias, ctr, out, B, H); break;
+    switch (L) {
+        LFM2Q_CONV(1)
+        LFM2Q_CONV(2)
+        LFM2Q_CONV(3)
+        LFM2Q_CONV(4)
+        LFM2Q_CONV(5)
+        LFM2Q_CONV(6)
+        LFM2Q_CONV(7)
+        LFM2Q_CONV(8)
+    default: return set_error(LFM2Q_ERR_SHAPE, "conv_step: need 1 <= L <= %d (%d)", CONV_MAX, L);
+    }
+#undef LFM2Q_CONV
+    return launch_status("conv_step");
 }

@@ -237,6 +237,26 @@ class DecodeOps:
                    v.data_ptr(), out.data_ptr(), B, nh, nkv, hd, max_len, float(scale), float(eps), ws.data_ptr(),
                    ws.numel() * 4, _capi.stream(qkv))
 
+    def conv_step(self, bcx, ring, wt, bias, ctr, out):
+        """One decode step of a gated short convolution (an addition): bcx [B, 3 H] = b | c | x, b x into row ctr[0] mod L
+        of ring [L, B, H], out [B, H] = c (conv of the ring with the taps wt [L, H] + bias), rounded as the bf16 tensor
+        ops (lfm2q_conv_step). Replaces the short-conv epilogue of gemv_epi(1, ...), kernels/lfm2_decode.cpp:130-150,
+        without its projection."""
+        for t, name in ((bcx, "bcx"), (ring, "ring"), (wt, "wt"), (out, "out")):
+            _check_bf16(t, name)
+        _check_t(ctr, torch.int64, "ctr")
+        if bias is not None:
+            _check_bf16(bias, "bias")
+        if ring.dim() != 3:
+            raise RuntimeError("conv_step: ring [L, B, H]")
+        L, B, H = ring.shape
+        if not (bcx.numel() == 3 * B * H and tuple(wt.shape) == (L, H) and out.numel() == B * H and ctr.numel() >= 1
+                and (bias is None or bias.numel() == H)):
+            raise RuntimeError("conv_step: bcx [B, 3H], ring [L, B, H], wt [L, H], out [B, H]")
+        _same_device(bcx, ring, wt, bias, ctr, out)
+        _capi.call("lfm2q_conv_step", bcx.data_ptr(), ring.data_ptr(), wt.data_ptr(), _capi.ptr(bias), ctr.data_ptr(),
+                   out.data_ptr(), B, H, L, _capi.stream(bcx))
+
     def _epi_args(self, W, scale, x, y, rows_per_out):
         _check_bf16(x, "x")
         _check_bf16(y, "y")

@@ -80,3 +80,35 @@ def test_attn_step_refuses_other_shapes(cuda):
                        ((4, 2, 64, 4096), "workspace")):
         with pytest.raises(RuntimeError, match=what):
             call(*args)
+
+
+@pytest.mark.parametrize("B,H,L,bias", [(1, 4, 3, False), (3, 252, 3, True), (1, 260, 1, False), (2, 512, 4, True),
+                                        (1, 2048, 8, True), (33, 1028, 2, False)])
+def test_conv_step_equals_the_bf16_ops(cuda, B, H, L, bias):
+    """L + 2 steps over a ring, the outputs and the ring equal to the bf16 tensor ops on the CPU: the products are
+    rounded alike and an fp32 sum of at most 8 of them differs by 2^-22 in another order, a tie apart: at most one
+    bf16 step (2^-8) of the sum."""
+    from lfm2opt.kernels import ext
+
+    bf = torch.bfloat16
+    g = torch.Generator().manual_seed(H + L)
+    wt = torch.randn(L, H, generator=g).to(bf)
+    b = torch.randn(H, generator=g).to(bf) if bias else None
+    ring = torch.randn(L, B, H, generator=g).to(bf)
+    dev = ring.to(cuda)
+    for pos in range(5, 7 + L):
+        bcx = torch.randn(B, 3 * H, generator=g).to(bf)
+        out = torch.empty(B, H, dtype=bf, device=cuda)
+        ext().conv_step(bcx.to(cuda), dev, wt.to(cuda), None if b is None else b.to(cuda),
+                        torch.tensor([pos, 0], device=cuda), out)
+        bb, cc, xx = bcx.chunk(3, -1)
+        ring[pos % L] = bb * xx
+        taps = torch.stack([wt[L - 1 - (pos - s) % L] for s in range(L)])
+        prod = ring * taps[:, None]
+        y = prod.float().sum(0).to(bf)
+        y = y if b is None else y + b
+        want = (cc * y).float()
+        assert torch.equal(dev.cpu(), ring)
+        step = 2.0 ** -7 * (cc.float() * prod.float().abs().sum(0)).abs()
+        assert ((out.cpu().float() - want).abs() <= step).all()
+        assert (out.cpu().float() != want).float().mean() <= 0.01
