@@ -189,6 +189,23 @@ size_t lfm2q_attn_step_workspace_bytes(int B, int n_heads, int n_kv, int max_len
 int lfm2q_conv_step(const lfm2q_bf16 *bcx, lfm2q_bf16 *ring, const lfm2q_bf16 *wt, const lfm2q_bf16 *bias,
                     const int64_t *ctr, lfm2q_bf16 *out, int B, int H, int L, lfm2q_stream_t stream);
 
+/* h bf16 [B, H] = the rows tok[b] of table bf16 [V, H] (NaN for a token outside it). H % 8 == 0, table and h 16-byte
+ * aligned. Replaces the embedding lookup of the reference's step (src/lfm2opt/runtime.py:246-250). */
+int lfm2q_embed_step(const lfm2q_bf16 *table, const int64_t *tok, lfm2q_bf16 *h, int B, int H, int V,
+                     lfm2q_stream_t stream);
+
+/* The end of a greedy decode step: copy fp32 [B, V] = logits (NULL: no copy), tok[b] = the index of the largest logit
+ * of row b whose block byte is 0 (blocked ones count as -inf; as torch.argmax: the lowest index among equals, NaN above
+ * all), row ctr[1] of out [max_new, B] = tok (not written outside it), ctr = ctr + (1, 1). With set_pos >= 0 the row is 0
+ * and ctr becomes (set_pos, 1): a prompt's first token. logits bf16 [B, V], V % 8 == 0, block [V] bytes; logits and copy
+ * 16-byte, block 8-byte aligned. ws: lfm2q_step_tail_workspace_bytes(), whose first 8 bytes are zero before the first
+ * call (each call leaves them so), not shared by overlapping calls.
+ * Replaces the argmax and counters of the reference's step (src/lfm2opt/runtime.py:127-139). */
+int lfm2q_step_tail(const lfm2q_bf16 *logits, const uint8_t *block, float *copy, int64_t *tok, int64_t *out,
+                    int64_t *ctr, int B, int V, int max_new, int set_pos, void *ws, size_t ws_bytes,
+                    lfm2q_stream_t stream);
+size_t lfm2q_step_tail_workspace_bytes(int B, int V);
+
 /* ------------------------------------------------------------------------------------------ W8A8 GEMM */
 
 /* Per-token activation quantization: s[r] = max(max_k |x[r, k]|, 1e-8) / 127 (IEEE division),

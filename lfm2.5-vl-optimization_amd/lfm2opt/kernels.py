@@ -257,6 +257,44 @@ class DecodeOps:
         _capi.call("lfm2q_conv_step", bcx.data_ptr(), ring.data_ptr(), wt.data_ptr(), _capi.ptr(bias), ctr.data_ptr(),
                    out.data_ptr(), B, H, L, _capi.stream(bcx))
 
+    def embed_step(self, table, tok, h):
+        """h [B, H] = rows tok [B] (int64) of table [V, H], bf16 (an addition; lfm2q_embed_step)."""
+        _check_bf16(table, "table")
+        _check_bf16(h, "h")
+        _check_t(tok, torch.int64, "tok")
+        if not (table.dim() == 2 and h.numel() == tok.numel() * table.shape[1]):
+            raise RuntimeError("embed_step: table [V, H], tok [B], h [B, H]")
+        _same_device(table, tok, h)
+        _capi.call("lfm2q_embed_step", table.data_ptr(), tok.data_ptr(), h.data_ptr(), tok.numel(), table.shape[1],
+                   table.shape[0], _capi.stream(h))
+
+    @staticmethod
+    def step_tail_workspace(B, V, device):
+        """A zeroed workspace for step_tail. Calls that share one must not overlap."""
+        n = _capi.lib().lfm2q_step_tail_workspace_bytes(B, V)
+        return torch.zeros(n // 8, dtype=torch.int64, device=device)
+
+    def step_tail(self, logits, block, copy, tok, out, ctr, ws, set_pos=-1):
+        """The end of a greedy decode step (an addition; lfm2q_step_tail): copy [B, V] fp32 (or None) = logits [B, V]
+        bf16, tok [B] = argmax of the logits not blocked (block [V] bool), row ctr[1] of out [max_new, B] = tok, ctr +=
+        1; with set_pos >= 0 row 0 and ctr = (set_pos, 1)."""
+        _check_bf16(logits, "logits")
+        _check_t(block, torch.bool, "block")
+        for t, name in ((tok, "tok"), (out, "out"), (ctr, "ctr"), (ws, "ws")):
+            _check_t(t, torch.int64, name)
+        if copy is not None:
+            _check_t(copy, torch.float32, "copy")
+        if not (logits.dim() == 2 and out.dim() == 2):
+            raise RuntimeError("step_tail: logits [B, V], out [max_new, B]")
+        B, V = logits.shape
+        if not (block.numel() == V and tok.numel() == B and out.shape[1] == B and ctr.numel() == 2
+                and (copy is None or copy.numel() == B * V)):
+            raise RuntimeError("step_tail: block [V], copy [B, V], tok [B], out [max_new, B], ctr [2]")
+        _same_device(logits, block, copy, tok, out, ctr, ws)
+        _capi.call("lfm2q_step_tail", logits.data_ptr(), block.data_ptr(), _capi.ptr(copy), tok.data_ptr(),
+                   out.data_ptr(), ctr.data_ptr(), B, V, out.shape[0], int(set_pos), ws.data_ptr(), ws.numel() * 8,
+                   _capi.stream(logits))
+
     def _epi_args(self, W, scale, x, y, rows_per_out):
         _check_bf16(x, "x")
         _check_bf16(y, "y")

@@ -112,3 +112,51 @@ def test_conv_step_equals_the_bf16_ops(cuda, B, H, L, bias):
         step = 2.0 ** -7 * (cc.float() * prod.float().abs().sum(0)).abs()
         assert ((out.cpu().float() - want).abs() <= step).all()
         assert (out.cpu().float() != want).float().mean() <= 0.01
+
+
+@pytest.mark.parametrize("B,V", [(1, 8), (1, 2048), (2, 2056), (9, 4096), (33, 65536), (70, 6000)])
+def test_step_tail_equals_the_torch_ops(cuda, B, V):
+    """Tokens, output row, counters and the fp32 copy equal copy_ / masked_fill_ / argmax / index_copy_ / add_, with ties
+    (within a chunk and across), blocked maxima, NaN, infinities and both zeros; the workspace serves every call."""
+    from lfm2opt.kernels import ext
+
+    E, g = ext(), torch.Generator().manual_seed(V)
+    ws = E.step_tail_workspace(B, V, cuda)
+    block = torch.zeros(V, dtype=torch.bool)
+    block[[0, V - 1, V // 2]] = True
+    ctr, out = torch.tensor([5, 0], device=cuda), torch.full((3, B), -1, device=cuda)
+    tok = torch.zeros(B, dtype=torch.long, device=cuda)
+    for row in range(5):
+        x = torch.randint(-8, 9, (B, V), generator=g).to(torch.bfloat16)  # many ties
+        if row == 1:
+            x[:, V // 2] = 100.0  # blocked
+        elif row == 2:
+            x[0] = float("-inf")
+            x[-1, torch.randint(V, (2,), generator=g)] = float("nan")
+        elif row == 3:
+            x = -x.abs()  # -0 and 0 tie
+            x[:, torch.randint(V, (V // 2,), generator=g)] = 0.0
+        copy = torch.empty(B, V, device=cuda)
+        E.step_tail(x.to(cuda), block.to(cuda), copy, tok, out, ctr, ws, set_pos=9 if row == 4 else -1)
+        want = x.float().masked_fill(block, float("-inf")).argmax(-1)
+        assert torch.equal(tok.cpu(), want)
+        assert torch.equal(copy.cpu().view(torch.int32), x.float().view(torch.int32))
+        if row < 3:
+            assert torch.equal(out[row].cpu(), want) and (out[row + 1:] == -1).all()
+        assert ctr.tolist() == ([9, 1] if row == 4 else [6 + row, 1 + row])
+    assert torch.equal(out[0].cpu(), want)  # the call with set_pos wrote row 0, the one at row 3 of 3 nothing
+
+
+@pytest.mark.parametrize("B,H", [(1, 8), (3, 520), (17, 2048)])
+def test_embed_step(cuda, B, H):
+    from lfm2opt.kernels import ext
+
+    g = torch.Generator().manual_seed(H)
+    table = torch.randn(100, H, generator=g).to(torch.bfloat16)
+    tok = torch.randint(100, (B,), generator=g)
+    h = torch.empty(B, H, dtype=torch.bfloat16, device=cuda)
+    ext().embed_step(table.to(cuda), tok.to(cuda), h)
+    assert torch.equal(h.cpu(), table[tok])
+    tok[-1] = 100
+    ext().embed_step(table.to(cuda), tok.to(cuda), h)
+    assert h[-1].isnan().all() and torch.equal(h[:-1].cpu(), table[tok[:-1]])
