@@ -206,6 +206,29 @@ int lfm2q_step_tail(const lfm2q_bf16 *logits, const uint8_t *block, float *copy,
                     lfm2q_stream_t stream);
 size_t lfm2q_step_tail_workspace_bytes(int B, int V);
 
+/* ------------------------------------------------------------------------------------------ prompt pass */
+
+/* Causal attention over a whole prompt at positions 0 .. T - 1: q / k head RMSNorm and rotary embedding of qkv bf16
+ * [B, T, (n_heads + 2 n_kv) head_dim] IN PLACE (fp32, rounded once), the keys and values into the caches k [B, n_kv,
+ * head_dim, max_len] and v [B, n_kv, max_len, head_dim], then out bf16 [B T, n_heads head_dim], or, with out NULL, its
+ * quantization as lfm2q_quant_groups writes it (oq int8, os fp32 [n_heads, B T]). Scores and sums in fp32, probabilities
+ * rounded to bf16. qk_w and rope as for lfm2q_attn_step (rope [>= T, 2, head_dim]); scale > 0, head_dim 64, n_heads / n_kv
+ * in {1, 2, 4, 8}, max_len >= T a multiple of 8, 16-byte aligned tensors. ws: lfm2q_prompt_attn_workspace_bytes(),
+ * contents irrelevant, not shared by overlapping calls.
+ * Replaces the prompt attention of the reference's prefill (src/lfm2opt/runtime.py:335-418). */
+int lfm2q_prompt_attn(lfm2q_bf16 *qkv, const float *qk_w, const float *rope, lfm2q_bf16 *k, lfm2q_bf16 *v,
+                      lfm2q_bf16 *out, int8_t *oq, float *os, int B, int T, int n_heads, int n_kv, int head_dim,
+                      int max_len, float scale, float eps, void *ws, size_t ws_bytes, lfm2q_stream_t stream);
+size_t lfm2q_prompt_attn_workspace_bytes(int B, int T, int n_kv);
+
+/* The gated short convolution over a whole prompt (zeros before it): of bcx bf16 [B, T, 3 H] = b | c | x, out bf16 [B T, H]
+ * = c (sum over the taps of (b x)[t - L + 1 + j] wt[j] + bias) with lfm2q_conv_step's roundings, or, with out NULL, its
+ * quantization as lfm2q_quant_groups writes it (oq int8, os fp32 [H / 64, B T], H % 64 == 0); ring bf16 [L, B, H] = the
+ * last L positions' b x, position p in row p mod L. wt bf16 [L, H], bias bf16 [H] or NULL; H % 8 == 0, 1 <= L <= 8,
+ * 16-byte aligned tensors. Replaces the short-conv prompt pass of the reference's prefill (src/lfm2opt/runtime.py:335-418). */
+int lfm2q_prompt_conv(const lfm2q_bf16 *bcx, const lfm2q_bf16 *wt, const lfm2q_bf16 *bias, lfm2q_bf16 *ring,
+                      lfm2q_bf16 *out, int8_t *oq, float *os, int B, int T, int H, int L, lfm2q_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------ W8A8 GEMM */
 
 /* Per-token activation quantization: s[r] = max(max_k |x[r, k]|, 1e-8) / 127 (IEEE division),

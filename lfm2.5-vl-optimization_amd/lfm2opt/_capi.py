@@ -25,7 +25,8 @@ class GemvOp(ctypes.Structure):
 
 # entry points that return something other than an int status
 RESTYPES = {"lfm2q_gemv_chain_workspace_bytes": ctypes.c_size_t, "lfm2q_gemm_workspace_bytes": ctypes.c_size_t,
-            "lfm2q_attn_step_workspace_bytes": ctypes.c_size_t, "lfm2q_step_tail_workspace_bytes": ctypes.c_size_t}
+            "lfm2q_attn_step_workspace_bytes": ctypes.c_size_t, "lfm2q_step_tail_workspace_bytes": ctypes.c_size_t,
+            "lfm2q_prompt_attn_workspace_bytes": ctypes.c_size_t}
 
 # name -> argument types (every entry point returns an int status unless listed in RESTYPES)
 SIGNATURES = {
@@ -41,6 +42,9 @@ SIGNATURES = {
     "lfm2q_embed_step": [_P, _P, _P, _I, _I, _I, _P],
     "lfm2q_step_tail": [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P],
     "lfm2q_step_tail_workspace_bytes": [_I, _I],
+    "lfm2q_prompt_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _F, _P, ctypes.c_size_t, _P],
+    "lfm2q_prompt_attn_workspace_bytes": [_I, _I, _I],
+    "lfm2q_prompt_conv": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "lfm2q_silu_mul": [_P, _P, _I, _I, _P],
     "lfm2q_quant_rows": [_P, _P, _P, _I, _I, _P],
     "lfm2q_quant_groups": [_P, _P, _P, _I, _I, _P],

@@ -295,6 +295,65 @@ class DecodeOps:
                    out.data_ptr(), ctr.data_ptr(), B, V, out.shape[0], int(set_pos), ws.data_ptr(), ws.numel() * 8,
                    _capi.stream(logits))
 
+    def prompt_attn(self, qkv, qk_w, rope, k, v, out, scale, eps):
+        """Causal attention over a whole prompt (an addition): qkv [B, T, (nh + 2 nkv) 64] normalized and rotated IN
+        PLACE, its keys and values into k [B, nkv, 64, max_len] / v [B, nkv, max_len, 64], out = bf16 [B T, nh 64] or
+        (int8 [B T, nh 64], scales [nh, B T]), the grouped input of the next W8A8 layer (lfm2q_prompt_attn). Replaces the
+        attention of the reference's prefill, src/lfm2opt/runtime.py:335-418."""
+        for t, name in ((qkv, "qkv"), (k, "k"), (v, "v")):
+            _check_bf16(t, name)
+        for t, name in ((qk_w, "qk_w"), (rope, "rope")):
+            _check_t(t, torch.float32, name)
+        if not (qkv.dim() == 3 and k.dim() == 4 and v.dim() == 4 and qk_w.dim() == 3):
+            raise RuntimeError("prompt_attn: qkv [B, T, (nh + 2 nkv) hd], k [B, nkv, hd, max_len], v [B, nkv, max_len, hd]")
+        B, T, W = qkv.shape
+        nkv, hd, max_len = k.shape[1:]
+        nh = qk_w.shape[1] - nkv
+        if not (W == (nh + 2 * nkv) * hd and tuple(qk_w.shape) == (2, nh + nkv, hd) and k.shape[0] == B
+                and tuple(v.shape) == (B, nkv, max_len, hd) and rope.numel() >= T * 2 * hd and T <= max_len):
+            raise RuntimeError("prompt_attn: qkv [B, T, (nh + 2 nkv) hd], qk_w [2, nh + nkv, hd], rope [>= T, 2, hd]")
+        y, q, s = self._prompt_out(out, B * T, nh * hd)
+        _same_device(qkv, qk_w, rope, k, v, y, q, s)
+        n = _capi.lib().lfm2q_prompt_attn_workspace_bytes(B, T, nkv)
+        ws = torch.empty(n, dtype=torch.uint8, device=qkv.device)
+        _capi.call("lfm2q_prompt_attn", qkv.data_ptr(), qk_w.data_ptr(), rope.data_ptr(), k.data_ptr(), v.data_ptr(),
+                   _capi.ptr(y), _capi.ptr(q), _capi.ptr(s), B, T, nh, nkv, hd, max_len, float(scale), float(eps),
+                   ws.data_ptr(), n, _capi.stream(qkv))
+
+    def prompt_conv(self, bcx, ring, wt, bias, out):
+        """The gated short convolution over a whole prompt (an addition): bcx [B, T, 3 H] = b | c | x, the last L
+        positions' b x into ring [L, B, H], out = bf16 [B T, H] or (int8 [B T, H], scales [H / 64, B T])
+        (lfm2q_prompt_conv). Replaces the short convolution of the reference's prefill, src/lfm2opt/runtime.py:335-418."""
+        for t, name in ((bcx, "bcx"), (ring, "ring"), (wt, "wt")):
+            _check_bf16(t, name)
+        if bias is not None:
+            _check_bf16(bias, "bias")
+        if not (bcx.dim() == 3 and ring.dim() == 3):
+            raise RuntimeError("prompt_conv: bcx [B, T, 3H], ring [L, B, H]")
+        B, T, W = bcx.shape
+        L, H = ring.shape[0], ring.shape[2]
+        if not (W == 3 * H and ring.shape[1] == B and tuple(wt.shape) == (L, H) and (bias is None or bias.numel() == H)):
+            raise RuntimeError("prompt_conv: bcx [B, T, 3H], ring [L, B, H], wt [L, H], bias [H]")
+        y, q, s = self._prompt_out(out, B * T, H)
+        _same_device(bcx, ring, wt, bias, y, q, s)
+        _capi.call("lfm2q_prompt_conv", bcx.data_ptr(), wt.data_ptr(), _capi.ptr(bias), ring.data_ptr(), _capi.ptr(y),
+                   _capi.ptr(q), _capi.ptr(s), B, T, H, L, _capi.stream(bcx))
+
+    @staticmethod
+    def _prompt_out(out, rows, cols):
+        """(bf16 output, int8 output, its scales), the absent ones None."""
+        if isinstance(out, tuple):
+            q, s = out
+            _check_t(q, torch.int8, "q")
+            _check_t(s, torch.float32, "s")
+            if not (cols % 64 == 0 and q.numel() == rows * cols and tuple(s.shape) == (cols // 64, rows)):
+                raise RuntimeError("output: int8 [rows, cols], scales [cols / 64, rows]")
+            return None, q, s
+        _check_bf16(out, "out")
+        if out.numel() != rows * cols:
+            raise RuntimeError("output: [rows, cols]")
+        return out, None, None
+
     def _epi_args(self, W, scale, x, y, rows_per_out):
         _check_bf16(x, "x")
         _check_bf16(y, "y")
