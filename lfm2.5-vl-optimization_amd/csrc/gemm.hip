@@ -14,6 +14,7 @@
 //   epilogue operands load during the current tile's epilogue) in 256 x 256, 256 x 128, 128 x 128 and 128 x 64
 //   tiles with 2-6 ring slots of 128-byte stages, optionally with K cut across workgroups through a workspace.
 // - gemm_w8_kernel: W8A16, bf16 activations x int8 weights on the bf16 matrix cores.
+// - gemm_i8_few_kernel: the grouped fold where the launch has few tiles (64 x 64, two groups a stage).
 // Which kernel and tile run is decided by the cost models of the dispatch section at the end of the file.
 //
 // M, N and K tails are zero-filled at load time by the buffer range check (K % 16 == 0); stores are predicated.
@@ -719,6 +720,132 @@ __global__ __launch_bounds__(GT * KSP) __attribute__((amdgpu_waves_per_eu(gemm_w
         epilogue<TM, TN, OUT>(acc, sx, sw, bias, Y, YsT, M, N, m0 + wm * WMt, n0 + wn * WNt, lane,
                               smem + wave * stage_bytes<TN>());
 }
+
+// ------------------------------------------------------------------------------------------------ grouped, few tiles
+// The grouped-64 fold of gemm_i8_kernel's GRP form (same operations in the same order: bit-identical) for launches whose 64
+// x 64 tiles leave a CU three or fewer: there a tile's time is the length of its chain of stages, not the machine's rate
+// (K = 8192 takes as long at 20 tokens as at 461). Against that kernel's 64 x 64 form: two groups per stage, so half the
+// barriers; each fold runs beside the next group's MFMAs (two int32 buffers), half of it after each; the next stage's
+// barrier and fragment reads come before a stage's arithmetic (two register sets). What is left bounds it: the weights' and
+// scales' latency from HBM (the loads alone take two thirds of the time) and ~32 vector operations a group. MI355X, us, 461
+// tokens x K x N: 8192 x 2048 31.5 -> 26.5, 2048 x 2048 10.2 -> 9.4, 2048 x 3072 (128 x 64 tiles before) 14.3 -> 11.8,
+// 2048 x 6144 (128 x 128) 20.8 -> 18.6. Deeper rings with one workgroup a CU (4 groups a stage, 6 or 8 slots), 8 wavefronts
+// of 32 x 16 blocks and 128-byte rows were no faster.
+template <int OUT>
+__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_i8_few_kernel(
+    const int8_t *__restrict__ X, const int8_t *__restrict__ W, const float *__restrict__ sxT,
+    const float *__restrict__ sw, const uint16_t *__restrict__ bias, void *__restrict__ Y, int M, int N, int K, int sh) {
+    constexpr int B = 64, G = 2, NST = 4;          // tile, groups per stage, ring slots
+    constexpr int PER = 2 * G + 1, TB = B * BK;    // loads per wavefront and stage, bytes of one operand's group
+    static_assert(G == 2 && NST % 2 == 0, "the register sets alternate with the slots, the int32 buffers with the groups");
+    static_assert(4 * stage_bytes<1>() <= NST * G * 2 * TB, "epilogue staging exceeds the LDS ring");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NST * G * (2 * TB + 256)];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    uint8_t(*sX)[G][TB] = reinterpret_cast<uint8_t(*)[G][TB]>(smem);
+    uint8_t(*sW)[G][TB] = reinterpret_cast<uint8_t(*)[G][TB]>(smem + NST * G * TB);
+    float(*sS)[G][B] = reinterpret_cast<float(*)[G][B]>(smem + 2 * NST * G * TB);
+    int tm, tn;
+    tile_of(blockIdx.x, (M + B - 1) / B, (N + B - 1) / B, tm, tn);
+    const int m0 = tm * B, n0 = tn * B;
+    const int KG = K / 64, S = (KG + G - 1) / G, F = KG / G;  // groups, stages, whole stages
+    const v4i rx = make_desc(X + (size_t)m0 * K, (uint32_t)std::min<long>((long)(M - m0) * K, 0x7fffffffL));
+    const v4i rw = make_desc(W + (size_t)n0 * K, (uint32_t)std::min<long>((long)(N - n0) * K, 0x7fffffffL));
+    const v4i rs = make_desc(sxT, (uint32_t)std::min<long>((long)KG * M * 4, 0x7fffffffL));
+    const int row = 16 * wave + (lane >> 2);  // of both operands: 16 rows per wavefront and group
+    const uint32_t off = (uint32_t)row * K + 16 * ((lane & 3) ^ ((row >> sh) & 3));
+    // stage st into ring slot `slot`; a group past K reads zeros and is not used
+    auto issue = [&](int st, int slot) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int k0 = (st * G + g) * 64;
+            const uint32_t vo = k0 < K ? off + k0 : 0xfffffff0u;
+            lds_dma16(rx, vo, lds_addr(sX[slot][g] + 1024 * wave));
+            lds_dma16(rw, vo, lds_addr(sW[slot][g] + 1024 * wave));
+        }
+        const int g = wave & 1;  // a group's 64 scales: two wavefronts load the same bytes to the same place
+        lds_dma4(rs, (uint32_t)(((long)(st * G + g) * M + m0 + lane) * 4), lds_addr(sS[slot][g]));
+    };
+    const int lr = lane & 31, lh = lane >> 5;
+    int fw[2], fx[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+        fw[kk] = swz(wn * 32 + lr, 2 * kk + lh, sh);
+        fx[kk] = swz(wm * 32 + lr, 2 * kk + lh, sh);
+    }
+    v16f facc[1][1];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) facc[0][0][e] = 0.f;
+    v16i ab[2] = {};
+    float pend = 0.f;  // the scale of the group in ab[1] that is still to be folded (first: 0 x 0)
+    auto fold = [&](int buf, float sc) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) facc[0][0][e] = __builtin_fmaf((float)ab[buf][e], sc, facc[0][0][e]);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) asm volatile("" : "+v"(facc[0][0][e]));  // folded here, not further down
+    };
+    struct Frag {
+        v4i w[2], x[2];
+        float sc;
+    };
+    Frag f[2][G];
+    auto mfma = [&](const Frag &d, int buf) {
+        const v16i zero = {};
+        ab[buf] = __builtin_amdgcn_mfma_i32_32x32x32_i8(d.w[0], d.x[0], zero, 0, 0, 0);
+        ab[buf] = __builtin_amdgcn_mfma_i32_32x32x32_i8(d.w[1], d.x[1], ab[buf], 0, 0, 0);
+    };
+    // stage st, visible to all, into a register set; everyone is done with the slot before it, which is refilled
+    auto fetch = [&](int st, int slot, Frag(&d)[G]) {
+        wait_stages<PER>(min(NST - 2, S - 1 - st));
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (st + NST - 1 < S) issue(st + NST - 1, (slot + NST - 1) % NST);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                d[g].w[kk] = *reinterpret_cast<const v4i *>(sW[slot][g] + fw[kk]);
+                d[g].x[kk] = *reinterpret_cast<const v4i *>(sX[slot][g] + fx[kk]);
+            }
+            d[g].sc = sS[slot][g][wm * 32 + lr];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int p = 0; p < NST - 1; ++p)
+        if (p < S) issue(p, p);
+    fetch(0, 0, f[0]);
+    auto step = [&](int st, auto slot_c) {
+        constexpr int SLOT = decltype(slot_c)::value;
+        if (st + 1 < S) fetch(st + 1, (SLOT + 1) % NST, f[(SLOT + 1) & 1]);
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            mfma(f[SLOT & 1][g], g);
+            fold(g ^ 1, pend);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {  // one MFMA, half of the fold
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            pend = f[SLOT & 1][g].sc;
+        }
+    };
+    int st = 0;
+    for (; st + NST <= F; st += NST) slot_steps<0, NST>(st, step);
+    slot_steps_below<0, NST - 1>(st, F, step);
+    fold(1, pend);
+    if (F < S) {  // an odd group count: the last stage's first group
+        const bool odd = F & 1;
+        Frag d = f[0][0];
+        if (odd) d = f[1][0];
+        mfma(d, 0);
+        fold(0, d.sc);
+    }
+    __syncthreads();  // every wavefront is done with the operand ring, which now holds the epilogue slices
+    epilogue<1, 1, OUT>(facc, nullptr, sw, bias, Y, nullptr, M, N, m0 + wm * 32, n0 + wn * 32, lane,
+                        smem + wave * stage_bytes<1>());
+}
+
 
 // LDS byte offset of 16-byte chunk c of a CPR-chunk row r: chunk c is stored at slot c ^ ((r / (8 / CPR * 2)) % CPR), so
 // the 16 rows a 16-lane phase of ds_read_b128 reads at one logical chunk hit 16 distinct bank groups (64 banks)
@@ -1763,6 +1890,18 @@ void launch_gemm_grouped(const int8_t *A, const int8_t *B, const float *sxT, con
         gemm_i8_kernel<128, 128, OUT, true, 3, 1, false, true><<<grid, GT, 0, st>>>(A, B, sxT, sw, bias, Y, M, N, K, sh,
                                                                                    YsT);
         return;
+    }
+    // bf16 output with K >= 2048 and at most three 64 x 64 tiles a CU: the kernel for few tiles, whatever tile the model
+    // above picks (it was fitted without it). Measured on MI355X over 18 such shapes 2 to 25 % faster (600 x 8192 x 2048 44.1
+    // -> 33.1 us, 1500 x 2048 x 2048 18.8 -> 18.4) but for 100 x 2048 x 16384 (15.2 -> 15.5); past three tiles a CU (600 x
+    // 2048 x 6144 21.0 -> 21.9) and for short K (1024 x 1152 x 1152 7.75 -> 8.2) it loses. LFM2Q_GEMM_GSEQ = 2 forces it.
+    if constexpr (!out_q8(OUT)) {
+        const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+        const bool forced = three || (knob_int(KNOB_GEMM_BM, 0) && knob_int(KNOB_GEMM_BN, 0));
+        if (gseq >= 0 ? gseq == 2 : !forced && K >= 2048 && t64 <= 3L * device_cus()) {
+            gemm_i8_few_kernel<OUT><<<dim3(t64), GT, 0, st>>>(A, B, sxT, sw, bias, Y, M, N, K, sh);
+            return;
+        }
     }
     LFM2Q_GEMM(128, 128)
     LFM2Q_GEMM(64, 128)

@@ -310,3 +310,25 @@ def test_grouped_argument_errors(E):
     with pytest.raises(RuntimeError, match="yq / ysT shape"):
         E.gemm_i8_q(xq, sxT, w64, sw64, None, yq64, torch.empty(2, 4, device="cuda"), False)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,K,N,bias,gelu", [(1, 64, 4, False, False), (63, 128, 64, True, False), (65, 192, 65, True, False),
+                                             (150, 448, 200, False, False), (130, 704, 72, True, True),
+                                             (20, 2112, 264, True, False)])
+def test_gemm_grouped_few_tiles(E, M, K, N, bias, gelu, tune):
+    """The few-tiles kernel (LFM2Q_GEMM_GSEQ = 2) at the edges of its tile, its two-group stages (odd group counts) and
+    its four-slot ring, bit-exact against the oracle (1 ulp through GELU, as the other forms)."""
+    tune("LFM2Q_GEMM_GSEQ", "2")
+    xq, sxT, wq, sw, b = operands(M + K + N, M, K, N, bias)
+    y = host_bits(run_grouped(E, xq, sxT, wq, sw, b, gelu))
+    u = int(ulp_dist(y, oracle.gemm_i8_grouped(xq, sxT, wq, sw, b, gelu)).max())
+    assert u <= (1 if gelu else 0), f"{u} bf16 ulp"
+
+
+def test_gemm_grouped_few_tiles_rounding_points(E, tune):
+    tune("LFM2Q_GEMM_GSEQ", "2")
+    xq, sxT, wq, sw, b, expect = rounding_cases.grouped_fold_case()
+    y = host_bits(run_grouped(E, xq, sxT, wq, sw, b, False))
+    for (m, n), bits in expect.items():
+        assert int(y[m, n]) == bits, (m, n, hex(int(y[m, n])))
+    assert np.array_equal(y, oracle.gemm_i8_grouped(xq, sxT, wq, sw, b))
