@@ -113,6 +113,12 @@ int lfm2q_gemv_rmsnorm(int wtype, int epi, const void *W, const float *scale, co
 int lfm2q_gemv_w4(int fmt, const void *Wq, const void *S, const int32_t *Z, const lfm2q_bf16 *x, lfm2q_bf16 *y,
                   int B, int N, int K, int group, int epi, lfm2q_stream_t stream);
 
+/* Batch-1 lfm2q_gemv_w4 of an RMS-normalized row, as lfm2q_gemv_rmsnorm: bit-identical to lfm2q_add_rmsnorm with no
+ * residual input followed by lfm2q_gemv_w4 with epi 0 or 1. h and norm_w bf16 [K], 128 <= K <= 2048. */
+int lfm2q_gemv_w4_rmsnorm(int fmt, const void *Wq, const void *S, const int32_t *Z, const lfm2q_bf16 *h,
+                          const lfm2q_bf16 *norm_w, float eps, lfm2q_bf16 *y, int N, int K, int group, int epi,
+                          lfm2q_stream_t stream);
+
 /* One GEMV of a chain: batch 1, int8 W [R, K] (R = N, or 2N = w1|w3 for epi 1) with fp32 scale [R], bf16 x [K],
  * bf16 y [N]. epi 0: y = bf16(acc * s); epi 1: the SwiGLU of lfm2q_gemv_swiglu; epi 2: y = bf16(y + bf16(acc * s))
  * in place (lfm2q_gemv_residual). */
@@ -250,6 +256,11 @@ int lfm2q_quant_groups(const lfm2q_bf16 *x, int8_t *q, float *sT, int rows, int 
  * add_rmsnorm_q (L = H): if y != NULL, h = bf16(h + y) in place; x = bf16(w * bf16(h * rs)),
  *   rs = 1 / sqrt(sum(h^2) / H + eps). Replaces launch_add_rmsnorm_q kernels/int8_gemm.cu:590-642 (binding
  *   add_rmsnorm_q(), kernels/int8_gemm.cpp:122-132). */
+/* add_rmsnorm_q's h and x without the INT8 row: h = bf16(h + y) in place if y != NULL, x bf16 [rows, H] as above
+ * (bit-identical). H % 8 == 0, H <= 8192, 16-byte aligned tensors. Replaces add_rmsnorm (kernels/lfm2_decode.cpp:33-38,
+ * kernel kernels/lfm2_decode.cu:96-121). */
+int lfm2q_add_rmsnorm(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm2q_bf16 *w, lfm2q_bf16 *x, int rows, int H, float eps,
+                      lfm2q_stream_t stream);
 int lfm2q_add_rmsnorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm2q_bf16 *w, int8_t *q, float *s,
                         lfm2q_bf16 *x, int rows, int H, float eps, int grouped, lfm2q_stream_t stream);
 /* add_layernorm_q (L = D): if y != NULL, h = bf16(h + y) in place; x = bf16(((h - mean) * rstd) * w + b),

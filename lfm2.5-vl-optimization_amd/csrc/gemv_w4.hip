@@ -18,6 +18,7 @@
 // Reference: kernels/lfm2_decode.cu:826-950 (gemv_w4_kernel, launch_gemv_w4), bound as gemv_w4 in
 // kernels/lfm2_decode.cpp:86-98; formats src/lfm2opt/quant.py:21-47 and src/lfm2opt/gptq.py:164-169.
 #include "common.hpp"
+#include "rmsnorm.hpp"
 #include "status.hpp"
 
 #include <algorithm>
@@ -83,6 +84,34 @@ __device__ __forceinline__ float epi_value(int epi, float a, float b, uint32_t h
     return rbf(silu_f32(rbf(a))) * rbf(b);
 }
 
+// The RMSNorm of a batch-1 row of K <= 2048 values inside the GEMV that reads it (NORM), bit-identical to add_rmsnorm_q's
+// x (rmsnorm.hpp): every wavefront that converts activations sums the whole row's squares in that kernel's order (lane l
+// takes vectors c 64 + l, zeros past K), beside its own chunk's loads, then applies the scale and the weight to its chunk.
+// Latency: the reduction delays the first products by ~1 us, the launch it saves takes 3.9 (three-layer INT4 steps 925 -> 781
+// us with it; lm_head alone 14.5 -> 14.0 us).
+template <bool NORM>
+struct RowNorm {
+    v4i hv[NORM ? 4 : 1];
+    __device__ __forceinline__ void issue(rsrc_t xr, int lane) {
+        if constexpr (NORM)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) hv[c] = buf_ld16(xr, (uint32_t)(c * 64 + lane) * 16u);
+    }
+    template <int V>
+    __device__ __forceinline__ void apply(const v4i *w, v4i (&x)[V], int K, float eps) const {
+        if constexpr (NORM) {
+            float ss = 0.f;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ss = sumsq8(hv[c], ss);
+            const float rs = rms_scale(wave_sum(ss), K, eps);
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[v][j] = (int)rms_apply2((uint32_t)w[v][j], (uint32_t)x[v][j], rs);
+        }
+    }
+};
+
 // ------------------------------------------------------------------------------------------------ batch 1
 // Persistent: about WPC wavefronts per CU, wavefront g handles output rows g, g + nw, ... Lane l owns the 16-byte
 // chunks (32 weights) c = l + 64 u, u < CPL, of every row; their activations stay in registers as bf16 pairs, with
@@ -90,10 +119,12 @@ __device__ __forceinline__ float epi_value(int epi, float a, float b, uint32_t h
 // sum_u s_u (dot_u - (128 + z_u) xs_u). The next NB - 1 rows' weights, scales and zero points are in flight while a
 // row is reduced; rows past the end go through an empty buffer range (zeros, no memory traffic). Chunks past K
 // (K < 2048 CPL) read zeros through the row's buffer range and have zero activations.
-template <int FMT, int CPL, int EPI>
+template <int FMT, int CPL, int EPI, bool NORM = false>
 __global__ __launch_bounds__(256) void gemv_w4_b1_kernel(const uint8_t *__restrict__ Wq, const void *__restrict__ S,
                                                          const int32_t *__restrict__ Z, const uint16_t *__restrict__ x,
-                                                         uint16_t *__restrict__ y, int N, int K, int group, int Sr) {
+                                                         uint16_t *__restrict__ y, int N, int K, int group, int Sr,
+                                                         const uint16_t *__restrict__ gain = nullptr, float eps = 0.f) {
+    static_assert(!NORM || CPL == 1, "the normalizing form holds K <= 2048");
     using F = W4Fmt<FMT>;
     const NibbleMasks nm;
     constexpr int NROW = EPI == EPI_SWIGLU ? 2 : 1;
@@ -138,13 +169,17 @@ __global__ __launch_bounds__(256) void gemv_w4_b1_kernel(const uint8_t *__restri
     __shared__ float xsq[CPL][4][64];
     const int jx = threadIdx.x >> 6;
     const rsrc_t xr = make_rsrc(x, (uint32_t)K * 2u);  // chunks past K read zeros (no branch around the loads)
-    v4i xd[CPL];
+    RowNorm<NORM> rn;
+    rn.issue(xr, lane);
+    v4i xd[CPL], xw[1];
 #pragma unroll
     for (int u = 0; u < CPL; ++u) xd[u] = buf_ld16(xr, (uint32_t)(lane + 64 * u) * 64u + 16u * jx);
+    if (NORM) xw[0] = buf_ld16(make_rsrc(gain, (uint32_t)K * 2u), (uint32_t)lane * 64u + 16u * jx);
     Item buf[NB];
 #pragma unroll
     for (int j = 0; j < NB - 1; ++j) load(buf[j], n + j * nw);
     __builtin_amdgcn_sched_barrier(0);
+    rn.apply(xw, xd, K, eps);
 #pragma unroll
     for (int u = 0; u < CPL; ++u) {
 #pragma unroll
@@ -233,10 +268,12 @@ __global__ __launch_bounds__(256) void gemv_w4_b1_kernel(const uint8_t *__restri
 // t + 256, ... with the same arithmetic into LDS (pair vector j of chunk c at xpv[j][c], its activation sum at
 // xsv[c]) -- and every lane reads its chunks' pairs from there, instead of every wavefront loading the whole row
 // and repacking it (same values, so the same bits).
-template <int FMT, int CPL, int EPI, int R, bool XS = false>
+template <int FMT, int CPL, int EPI, int R, bool XS = false, bool NORM = false>
 __global__ __launch_bounds__(256) void gemv_w4_b1o_kernel(const uint8_t *__restrict__ Wq, const void *__restrict__ S,
                                                           const int32_t *__restrict__ Z, const uint16_t *__restrict__ x,
-                                                          uint16_t *__restrict__ y, int N, int K, int group, int Sr) {
+                                                          uint16_t *__restrict__ y, int N, int K, int group, int Sr,
+                                                          const uint16_t *__restrict__ gain = nullptr, float eps = 0.f) {
+    static_assert(!NORM || CPL == 1, "the normalizing form holds K <= 2048");
     using F = W4Fmt<FMT>;
     const NibbleMasks nm;
     constexpr int NROW = EPI == EPI_SWIGLU ? 2 : 1;
@@ -255,13 +292,19 @@ __global__ __launch_bounds__(256) void gemv_w4_b1o_kernel(const uint8_t *__restr
     // activations first (cache hits), then every row's weights, scales and zero points; the activations of chunk c
     // are bytes 64 c .. 64 c + 63 of x (chunks past K read zeros through the range)
     const rsrc_t xr = make_rsrc(x, (uint32_t)K * 2u);
-    v4i xd[CPT][4];
+    v4i xd[CPT][4], xw[4];
+    RowNorm<NORM> rn;
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
         const int c = XS ? (int)threadIdx.x + 256 * u : lane + 64 * u;
-        if (!XS || NC % 256 == 0 || c < NC)
+        if (!XS || NC % 256 == 0 || c < NC) {  // (uniform in a wavefront)
+            rn.issue(xr, lane);
 #pragma unroll
             for (int j = 0; j < 4; ++j) xd[u][j] = buf_ld16(xr, (uint32_t)c * 64u + 16u * j);
+            if (NORM)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) xw[j] = buf_ld16(make_rsrc(gain, (uint32_t)K * 2u), (uint32_t)c * 64u + 16u * j);
+        }
     }
     v4i w[R][NROW][CPL];
     uint32_t sr[R][NROW][CPL], zr[R][NROW][CPL];
@@ -306,6 +349,7 @@ __global__ __launch_bounds__(256) void gemv_w4_b1o_kernel(const uint8_t *__restr
             if (NC % 256 == 0 || c < NC) {
                 uint32_t pp[16];
                 float sum;
+                rn.apply(xw, xd[u], K, eps);
                 repack(xd[u], pp, sum);
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
@@ -326,7 +370,10 @@ __global__ __launch_bounds__(256) void gemv_w4_b1o_kernel(const uint8_t *__restr
         }
     } else {
 #pragma unroll
-        for (int u = 0; u < CPL; ++u) repack(xd[u], xp[u], xs[u]);
+        for (int u = 0; u < CPL; ++u) {
+            rn.apply(xw, xd[u], K, eps);
+            repack(xd[u], xp[u], xs[u]);
+        }
     }
     float part[V];
 #pragma unroll
@@ -560,9 +607,9 @@ __global__ __launch_bounds__(64 * NWK) void gemv_w4_mfma_kernel(const uint8_t *_
 }
 
 // ------------------------------------------------------------------------------------------------ dispatch
-template <int FMT, int EPI>
+template <int FMT, int EPI, bool NORM = false>
 void launch_w4_b1(const uint8_t *W, const void *S, const int32_t *Z, const uint16_t *x, uint16_t *y, int N, int K,
-                  int group, hipStream_t st) {
+                  int group, hipStream_t st, const uint16_t *gain = nullptr, float eps = 0.f) {
     // wavefronts per CU: 4 up to 3072 rows (each wavefront amortizes its activation repack over more rows), 16 from
     // 32768 rows (more loads in flight on a long stream), else 8; the LFM2Q_W4_WPC knob overrides it
     const int wpc_env = knob_int(KNOB_W4_WPC, 0);
@@ -588,12 +635,14 @@ void launch_w4_b1(const uint8_t *W, const void *S, const int32_t *Z, const uint1
 #define LFM2Q_W4O(C_)                                                                                 \
     do {                                                                                              \
         if (xs)                                                                                       \
-            gemv_w4_b1o_kernel<FMT, C_, EPI, 2, true><<<go, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N); \
+            gemv_w4_b1o_kernel<FMT, C_, EPI, 2, true, NORM><<<go, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N, gain, eps); \
         else                                                                                          \
-            gemv_w4_b1o_kernel<FMT, C_, EPI, 2><<<go, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N);   \
+            gemv_w4_b1o_kernel<FMT, C_, EPI, 2, false, NORM><<<go, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N, gain, eps); \
     } while (0)
         if (C <= 64)
             LFM2Q_W4O(1);
+        else if constexpr (NORM)
+            ;  // the entry point admits K <= 2048 only
         else if (C <= 128)
             LFM2Q_W4O(2);
         else
@@ -602,7 +651,9 @@ void launch_w4_b1(const uint8_t *W, const void *S, const int32_t *Z, const uint1
         return;
     }
     if (C <= 64)
-        gemv_w4_b1_kernel<FMT, 1, EPI><<<grid, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N);
+        gemv_w4_b1_kernel<FMT, 1, EPI, NORM><<<grid, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N, gain, eps);
+    else if constexpr (NORM)
+        ;
     else if (C <= 128)
         gemv_w4_b1_kernel<FMT, 2, EPI><<<grid, 256, 0, st>>>(W, S, Z, x, y, N, K, group, N);
     else
@@ -722,4 +773,30 @@ extern "C" int lfm2q_gemv_w4(int fmt, const void *Wq, const void *S, const int32
     }
 #undef LFM2Q_W4RUN
     return launch_status("gemv_w4");
+}
+
+extern "C" int lfm2q_gemv_w4_rmsnorm(int fmt, const void *Wq, const void *S, const int32_t *Z, const lfm2q_bf16 *h,
+                                     const lfm2q_bf16 *norm_w, float eps, lfm2q_bf16 *y, int N, int K, int group, int epi,
+                                     lfm2q_stream_t stream) {
+    LFM2Q_REQUIRE(fmt == 0 || fmt == 1, LFM2Q_ERR_ARG, "gemv_w4_rmsnorm: fmt must be 0 or 1, got %d", fmt);
+    LFM2Q_REQUIRE(epi == 0 || epi == 1, LFM2Q_ERR_ARG, "gemv_w4_rmsnorm: epi must be 0 (none) or 1 (SwiGLU)");
+    LFM2Q_REQUIRE(Wq && S && h && norm_w && y && (fmt == 0 || Z), LFM2Q_ERR_ARG, "gemv_w4_rmsnorm: null pointer");
+    LFM2Q_REQUIRE(N >= 1 && K >= 128 && K <= 2048, LFM2Q_ERR_SHAPE,
+                  "gemv_w4_rmsnorm: need N >= 1 and 128 <= K <= 2048 (N=%d K=%d)", N, K);
+    LFM2Q_REQUIRE(group >= 32 && group % 32 == 0 && K % group == 0, LFM2Q_ERR_SHAPE,
+                  "gemv_w4_rmsnorm: group size must be a multiple of 32 dividing K (group=%d K=%d)", group, K);
+    LFM2Q_REQUIRE(aligned16(Wq) && aligned16(h) && aligned16(norm_w), LFM2Q_ERR_ALIGN,
+                  "gemv_w4_rmsnorm: Wq, h and norm_w must be 16-byte aligned");
+    const uint8_t *W = reinterpret_cast<const uint8_t *>(Wq);
+    const hipStream_t st = (hipStream_t)stream;
+#define LFM2Q_W4N(F_, E_) launch_w4_b1<F_, E_, true>(W, S, Z, h, y, N, K, group, st, norm_w, eps)
+    if (fmt == 0) {
+        if (epi == 0) LFM2Q_W4N(0, EPI_NONE);
+        else LFM2Q_W4N(0, EPI_SWIGLU);
+    } else {
+        if (epi == 0) LFM2Q_W4N(1, EPI_NONE);
+        else LFM2Q_W4N(1, EPI_SWIGLU);
+    }
+#undef LFM2Q_W4N
+    return launch_status("gemv_w4_rmsnorm");
 }

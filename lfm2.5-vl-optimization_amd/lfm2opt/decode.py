@@ -208,13 +208,16 @@ class DecodeLinears:
 
     def norm_fusable(self, B, key):
         """Whether the linear for key at batch B runs as one GEMV that also computes its input's RMSNorm
-        (gemv_rmsnorm): batch 1 on the GEMV path, INT8 or BF16 weights, K a supported chunk multiple."""
+        (gemv_rmsnorm, gemv_w4_rmsnorm): batch 1 on the GEMV path, K a chunk multiple the INT8 or BF16 kernel takes, or
+        INT4 weights of K <= 2048 with no AWQ scaling of their input."""
         if not (self.norm_fusion and B == 1 and self.path(B, key) == "gemv"):
             return False
         fmt = self.fmt(key)
         K = self.shape(key)[1]
         if fmt == "int8":
             return K in (1024, 2048, 4096, 8192)
+        if fmt == "int4":
+            return 128 <= K <= 2048 and K % 8 == 0 and key not in self.lin_inv_s
         return fmt == "bf16" and K in (512, 1024, 2048, 4096)
 
     def linear_normed(self, h, key, norm_w, eps, swiglu=False, out=None):
@@ -224,6 +227,10 @@ class DecodeLinears:
         N = w.shape[0] // 2 if swiglu else w.shape[0]
         y = out if out is not None else torch.empty(1, N, device=h.device, dtype=h.dtype)
         self.last_path = "gemv"
+        if w.dtype in (torch.uint8, torch.int32):
+            self.K.gemv_w4_rmsnorm(w, self.lin_scale[key], self.lin_zeros.get(key), h.contiguous(), norm_w, eps, y,
+                                   1 if swiglu else 0)
+            return y
         self.K.gemv_rmsnorm(w, self.lin_scale.get(key), h.contiguous(), norm_w, eps, y, 1 if swiglu else 0)
         return y
 

@@ -201,6 +201,46 @@ class DecodeOps:
         _capi.call("lfm2q_gemv_rmsnorm", 0 if int8 else 1, int(epi), W.data_ptr(), _capi.ptr(scale), h.data_ptr(),
                    norm_w.data_ptr(), float(eps), y.data_ptr(), N, K, _capi.stream(h))
 
+    def gemv_w4_rmsnorm(self, Wp, S, zeros, h, norm_w, eps, y, epi=0):
+        """The batch-1 INT4 GEMV of RMSNorm(h) (an addition), as gemv_rmsnorm: Wp, S as in gemv_w4 (zeros None) or
+        gemv_w4z; epi 0 or 1 (SwiGLU). Bit-identical to add_rmsnorm (no residual input), then that GEMV. 128 <= K <= 2048."""
+        for t, name in ((h, "h"), (norm_w, "norm_w"), (y, "y")):
+            _check_bf16(t, name)
+        fmt, per = (0, 2) if zeros is None else (1, 8)
+        wdt, sdt = (torch.uint8, torch.float32) if fmt == 0 else (torch.int32, torch.float16)
+        _check_t(Wp, wdt, "Wp")
+        _check_t(S, sdt, "S")
+        if epi not in (0, 1) or Wp.dim() != 2:
+            raise RuntimeError("gemv_w4_rmsnorm: Wp [R, K / 2] or [R, K / 8], epi 0 (none) or 1 (swiglu)")
+        R, K = Wp.size(0), Wp.size(1) * per
+        group = self._w4_group(S, R, K)
+        if fmt == 1:
+            _check_t(zeros, torch.int32, "zeros")
+            if tuple(zeros.shape) != (R, (K // group + 7) // 8):
+                raise RuntimeError("qzeros: contiguous int32 [N, ceil(K/group/8)]")
+        N = R // 2 if epi == 1 else R
+        if (epi == 1 and R % 2) or h.numel() != K or norm_w.numel() != K or y.numel() != N:
+            raise RuntimeError("gemv_w4_rmsnorm: h [1, K], norm_w [K], y [1, N] (batch 1)")
+        _same_device(Wp, S, zeros, h, norm_w, y) if fmt == 1 else _same_device(Wp, S, h, norm_w, y)
+        _capi.call("lfm2q_gemv_w4_rmsnorm", fmt, Wp.data_ptr(), S.data_ptr(), _capi.ptr(zeros), h.data_ptr(),
+                   norm_w.data_ptr(), float(eps), y.data_ptr(), N, K, group, int(epi), _capi.stream(h))
+
+    def add_rmsnorm(self, h, y, w, x, eps):
+        """h += y (optional, in place, bf16-rounded); x = bf16(w * bf16(rmsnorm(h))): add_rmsnorm_q's h and x without the
+        INT8 row. Reference: add_rmsnorm(), kernels/lfm2_decode.cpp:33-38."""
+        for t, name in ((h, "h"), (w, "w"), (x, "x")):
+            _check_bf16(t, name)
+        H = h.size(-1)
+        if not (w.numel() == H and H % 8 == 0 and 0 < H <= 8192 and h.numel() > 0 and x.numel() == h.numel()):
+            raise RuntimeError("add_rmsnorm: h, x [rows, H], w [H] (H % 8 == 0, H <= 8192)")
+        if y is not None:
+            _check_bf16(y, "y")
+            if y.numel() != h.numel():
+                raise RuntimeError("y shape")
+        _same_device(h, y, w, x)
+        _capi.call("lfm2q_add_rmsnorm", h.data_ptr(), _capi.ptr(y), w.data_ptr(), x.data_ptr(), h.numel() // H, H,
+                   float(eps), _capi.stream(h))
+
     def gemv_residual(self, W, scale, x, h):
         """h [B, N] += bf16(x @ W^T * scale) in place, rounded as the reference's residual add
         (kernels/lfm2_decode.cu:108-113): h = bf16(h + bf16(acc * s))."""

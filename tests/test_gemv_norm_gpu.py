@@ -151,3 +151,45 @@ def test_runtime_step_fused_norms_bit_identical(cuda, monkeypatch):
         got[fuse] = (step_logits(dec, ids, graph=True), step_logits(dec, ids, graph=False))
     assert torch.equal(got["1"][0], got["1"][1]), "graph replays differ from eager steps"
     assert torch.equal(got["1"][0], got["0"][0]), "fused norms change the logits"
+
+
+@pytest.mark.parametrize("rows,H,res", [(1, 72, False), (3, 2048, True), (17, 2048, False), (5, 8192, True), (2, 1000, True)])
+def test_add_rmsnorm_equals_add_rmsnorm_q(E, E8, rows, H, res):
+    """h and x bit for bit those of add_rmsnorm_q."""
+    g = torch.Generator().manual_seed(rows + H)
+    h = torch.randn(rows, H, generator=g).to(torch.bfloat16).cuda()
+    y = torch.randn(rows, H, generator=g).to(torch.bfloat16).cuda() if res else None
+    w = (torch.rand(H, generator=g) + 0.5).to(torch.bfloat16).cuda()
+    h2, x, x2 = h.clone(), torch.empty_like(h), torch.empty_like(h)
+    q, s = torch.empty(rows, H, device="cuda", dtype=torch.int8), torch.empty(rows, device="cuda")
+    E8.add_rmsnorm_q(h2, y, w, q, s, 1e-5, x=x2)
+    E.add_rmsnorm(h, y, w, x, 1e-5)
+    assert torch.equal(x, x2) and torch.equal(h, h2)
+
+
+@pytest.mark.parametrize("fmt", [0, 1])
+@pytest.mark.parametrize("R,epi", [(6, 0), (3072, 0), (32768, 0), (65536, 0), (16384, 1), (40, 1)])
+@pytest.mark.parametrize("K,group", [(2048, 128), (1024, 64), (128, 32), (1120, 32)])
+def test_gemv_w4_rmsnorm_equals_norm_then_gemv(E, E8, fmt, R, epi, K, group, tune):
+    """Bit-identical to add_rmsnorm, then the INT4 GEMV, one-shot and persistent (32768 weight rows and more), with whole
+    and partial rows of chunks."""
+    g = torch.Generator().manual_seed(R + K + fmt)
+    G = K // group
+    if fmt == 0:
+        W = torch.randint(0, 256, (R, K // 2), generator=g, dtype=torch.uint8).cuda()
+        S, Z = (torch.rand(R, G, generator=g) * 0.01).cuda(), None
+    else:
+        W = torch.randint(-2**31, 2**31 - 1, (R, K // 8), generator=g, dtype=torch.int64).to(torch.int32).cuda()
+        S = (torch.rand(R, G, generator=g) * 0.01).half().cuda()
+        Z = torch.randint(0, 2**31 - 1, (R, (G + 7) // 8), generator=g, dtype=torch.int64).to(torch.int32).cuda()
+    h, nw = row(g, K), (torch.rand(K, generator=g) + 0.5).to(torch.bfloat16).cuda()
+    x = torch.empty_like(h)
+    E.add_rmsnorm(h, None, nw, x, 1e-5)
+    ref = torch.empty(1, R // 2 if epi else R, device="cuda", dtype=torch.bfloat16)
+    y = torch.empty_like(ref)
+    if fmt == 0:
+        E.gemv_w4(W, S, x, ref, epi=epi)
+    else:
+        E.gemv_w4z(W, S, Z, x, ref, epi=epi)
+    E.gemv_w4_rmsnorm(W, S, Z, h, nw, 1e-5, y, epi)
+    assert np.array_equal(host_bits(y), host_bits(ref))
