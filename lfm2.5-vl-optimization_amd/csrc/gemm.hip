@@ -1932,11 +1932,48 @@ void launch_gemm_bf16a(const uint16_t *X, const int8_t *B, const float *sx, cons
 #undef LFM2Q_GEMM
 }
 
+// W8A16 tile and in-workgroup K split. A tile's time is its stages' (64 k per group), each as long as the direct loads in
+// flight on the CU take: with `per` tiles on the busiest CU, `resident` of them at a time, time = (stages x the stage time
+// at the number resident) summed over the rounds + round x rounds + call. Fitted (us) to MI355X timings of the nine
+// configurations on 112 shapes (20 to 4000 rows over the LFM2 and SigLIP2 weights): within 5 % of a timing (rms), its pick
+// within 0.3 % of the fastest on average, where the W8A8 table above gave 3.7 % and up to 32 % (4000 x 4304 x 1152 97.6 ->
+// 73.8 us, 4000 x 1152 x 3456 58.0 -> 47.2, 1500 x 2048 x 2048 27.8 -> 25.5).
+struct W8Cfg {
+    int bm, bn, ksp, resident;
+    double stage[4], round, call;
+};
+inline W8Cfg pick_w8(int M, int N, int K) {
+    static const W8Cfg opts[] = {{64, 64, 1, 4, {0.465, 0.574, 0.758, 0.888}, 0.0, 3.665},
+                                 {64, 64, 2, 2, {0.602, 0.988}, 0.237, 3.893},
+                                 {64, 64, 4, 1, {1.036}, 1.774, 1.815},
+                                 {64, 128, 1, 3, {0.561, 0.797, 1.093}, 0.0, 4.193},
+                                 {64, 128, 2, 1, {0.842}, 2.769, 1.651},
+                                 {128, 64, 1, 2, {0.604, 0.749}, 0.831, 3.061},
+                                 {128, 64, 2, 1, {0.834}, 2.088, 1.917},
+                                 {128, 128, 1, 2, {0.765, 1.116}, 2.269, 2.421},
+                                 {128, 128, 2, 1, {1.217}, 4.286, 0.705}};
+    const long cus = device_cus();
+    double best = 1e300;
+    W8Cfg bestc = opts[0];
+    for (const W8Cfg &o : opts) {
+        const long tiles = (long)((M + o.bm - 1) / o.bm) * ((N + o.bn - 1) / o.bn), per = (tiles + cus - 1) / cus;
+        const long full = per / o.resident, rest = per % o.resident;
+        const int stages = ((K + 63) / 64 + o.ksp - 1) / o.ksp;
+        double t = o.call + o.round * (double)(full + (rest ? 1 : 0)) + (double)full * stages * o.stage[o.resident - 1];
+        if (rest) t += stages * o.stage[rest - 1];
+        if (t < best) {
+            best = t;
+            bestc = o;
+        }
+    }
+    return bestc;
+}
+
 template <int OUT>
 void launch_gemm_w8(const uint16_t *X, const int8_t *W, const float *sw, const uint16_t *bias, uint16_t *Y, int M,
                     int N, int K, hipStream_t st, void *ws = nullptr, size_t ws_bytes = 0) {
-    const TileCfg t = pick_tile(M, N, K, TILES_GROUPED);
-    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    TileCfg t = pick_tile(M, N, K, TILES_GROUPED);
+    long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int KT = (K + 63) / 64;
     // With a workspace, K slices over workgroups where the tiles leave more than half the CUs idle: SK = CUs / tiles,
     // at most 8 and with at least 2048 k per slice (shorter slices lost to the unsplit kernel on MI355X: w1|w3 at 64
@@ -1950,12 +1987,21 @@ void launch_gemm_w8(const uint16_t *X, const int8_t *W, const float *sw, const u
         while (sk > 1 && 4 * (size_t)SPLIT_CNT_WORDS + (size_t)tiles * sk * t.bm * t.bn * 4 > std::min(ws_bytes, GEMM_SPLIT_BYTES)) --sk;
         if (tiles > (long)SPLIT_CNT_WORDS || sk < 2) sk = 1;
     }
+    // without that split, the tile and the split inside the workgroup by W8A16's own model
+    const bool own = sk == 1 && !(knob_int(KNOB_GEMM_BM, 0) && knob_int(KNOB_GEMM_BN, 0));
+    const W8Cfg c = pick_w8(M, N, K);
+    if (own) {
+        t.bm = c.bm;
+        t.bn = c.bn;
+        tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    }
     const dim3 grid(tiles * sk);
-    // K split inside the workgroup where the tiles leave at most one workgroup per CU (a lone workgroup of 4
-    // wavefronts is bound by its LDS -> convert -> MFMA chain): 4 groups for 64 x 64 tiles, 2 for the others (LDS).
+    // With a split over workgroups or a forced tile, K split inside the workgroup where the tiles leave at most one
+    // workgroup per CU (a lone workgroup of 4 wavefronts keeps too few loads in flight): 4 groups for 64 x 64 tiles, 2 for
+    // the others (LDS).
     // The LFM2Q_GEMM_KSPLIT knob (1 / 2 / 4) forces it (4 only for 64 x 64).
     const bool s64 = t.bm == 64 && t.bn == 64;
-    int ksp = ((long)grid.x <= device_cus() && KT / sk >= 8) ? (s64 ? 4 : 2) : 1;
+    int ksp = own ? c.ksp : ((long)grid.x <= device_cus() && KT / sk >= 8) ? (s64 ? 4 : 2) : 1;
     if (const int f = knob_int(KNOB_GEMM_KSPLIT, 0)) ksp = f == 4 && s64 ? 4 : f == 2 ? 2 : 1;
     uint32_t *const w = static_cast<uint32_t *>(ws);
     if (sk > 1) {
