@@ -6,11 +6,14 @@ are valid in the library. There is no fallback: if the library is missing, every
 """
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import pathlib
 
 import torch  # noqa: F401  (must precede the dlopen below, see module docstring)
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent.parent / "lib" / "liblfm2q.so"
+NATIVE_PATH = LIB_PATH.with_name("_lfm2q_native.so")
 
 _P = ctypes.c_void_p
 _I = ctypes.c_int
@@ -91,6 +94,27 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The CPython module of the eager ops (binding/native.cpp), which checks their arguments and calls liblfm2q without
+    ctypes. Like the library it has no fallback."""
+    global _native
+    if _native is None:
+        lib()  # the same shared object, opened by its path first
+        if not NATIVE_PATH.exists():
+            raise RuntimeError(f"_lfm2q_native.so is not built ({NATIVE_PATH}); build it with "
+                               f"`make -C lfm2.5-vl-optimization_amd/binding` or __graft_entry__.build()")
+        spec = importlib.util.spec_from_loader(
+            "_lfm2q_native", importlib.machinery.ExtensionFileLoader("_lfm2q_native", str(NATIVE_PATH)))
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        m.set_workspaces(_workspaces, prepare_workspace)
+        _native = m
+    return _native
+
+
 def call(name, *args):
     """Call entry point `name`; a non-zero status becomes RuntimeError with the library's message."""
     st = getattr(lib(), name)(*args)
@@ -112,7 +136,7 @@ def get_tuning(name):
 
 def stream(t):
     """Raw hipStream_t of torch's current stream on t's device (the reference launches on the same stream)."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def ptr(t):

@@ -81,6 +81,11 @@ def linear_path(mode, fmt, B, N, K, has_bf16):
     return "gemv" if B <= (48 if N >= HEAD_ROWS else 24 if N >= W8A16_MIN_ROWS else GEMV_MAX_BATCH_NARROW) else "linear"
 
 
+# per stored dtype: the weight format, and the input channels of one element
+_FMT = {torch.bfloat16: "bf16", torch.int8: "int8", torch.uint8: "int4", torch.int32: "int4"}
+_PACK = {torch.bfloat16: 1, torch.int8: 1, torch.uint8: 2, torch.int32: 8}
+
+
 class DecodeLinears:
     """The decode linears of one model, keyed like the reference's `lin` dict (("qkv", i), ("w13", i), ("head", 0),
     ...; w1|w3 stacked as one [2 I, K] matrix under a "w13" key).
@@ -144,17 +149,17 @@ class DecodeLinears:
 
     # ---- dispatch -----------------------------------------------------------------------------------------------
     def fmt(self, key):
-        dt = self.lin[key].dtype
-        return "bf16" if dt == torch.bfloat16 else "int8" if dt == torch.int8 else "int4"
+        return _FMT[self.lin[key].dtype]
 
     def shape(self, key):
         """(N, K) of the weight behind key."""
         w = self.lin[key]
-        return w.shape[0], w.shape[1] * {torch.bfloat16: 1, torch.int8: 1, torch.uint8: 2, torch.int32: 8}[w.dtype]
+        return w.shape[0], w.shape[1] * _PACK[w.dtype]
 
     def path(self, B, key):
-        N, K = self.shape(key)
-        return linear_path(self.mode, self.fmt(key), B, N, K, key in self.lin_bf16)
+        w = self.lin[key]
+        N, K = w.shape
+        return linear_path(self.mode, _FMT[w.dtype], B, N, K * _PACK[w.dtype], key in self.lin_bf16)
 
     def _bf16_weight(self, key):
         w = self.lin[key]
@@ -188,7 +193,7 @@ class DecodeLinears:
         if p == "w8a16":
             y = self.w8[key](x)
             return y if bias is None else y + bias
-        y = torch.empty(B, self.lin[key].shape[0], device=x.device, dtype=x.dtype)
+        y = x.new_empty((B, self.lin[key].shape[0]))
         self._gemv(x.contiguous(), key, y, 0)
         return y if bias is None else y + bias
 

@@ -43,7 +43,7 @@ class DecodeOps:
     """Decode-path ops (reference: kernels/lfm2_decode.cpp)."""
 
     def __init__(self):
-        _capi.lib()
+        self._n = _capi.native()
         self.pdl = True
         self.gemv_impl = 1
 
@@ -51,27 +51,7 @@ class DecodeOps:
     def gemv(self, W, scale, x, y, rows=0):
         """y [B, N] = x [B, K] @ W^T, W [N, K] bf16 or int8 (then scale [N] fp32 is required); any B >= 1.
         Reference: gemv(), kernels/lfm2_decode.cpp:74-85. rows: output rows per wavefront for B == 1."""
-        _check_bf16(x, "x")
-        _check_bf16(y, "y")
-        if not (W.is_cuda and W.is_contiguous() and W.dim() == 2):
-            raise RuntimeError("W must be a contiguous CUDA matrix")
-        int8 = W.dtype == torch.int8
-        if not (int8 or W.dtype == torch.bfloat16):
-            raise RuntimeError("W must be bf16 or int8")
-        if int8 and (scale is None or scale.dtype != torch.float32):
-            raise RuntimeError("int8 W needs fp32 scale")
-        N, K = W.shape
-        B = x.numel() // K if K else 0
-        if not (B >= 1 and x.numel() == B * K and y.numel() == B * N):
-            raise RuntimeError("x [B, K], y [B, N]")
-        if scale is not None:
-            _check_t(scale, torch.float32, "scale")
-            if scale.numel() != N:
-                raise RuntimeError("scale must have N elements")
-        _same_device(W, x, y, scale)
-        fn = "lfm2q_gemv_w8" if int8 else "lfm2q_gemv_bf16"
-        _capi.call(fn, W.data_ptr(), _capi.ptr(scale), x.data_ptr(), y.data_ptr(), B, N, K, int(rows),
-                   _capi.stream(x))
+        self._n.gemv(W, scale, x, y, int(rows))
 
     def gemv_epi(self, epi, W, scale, x, y, state=None, cw=None, cbias=None):
         """epi 0: W = w1|w3 [2S, K] -> y [B, S] = silu(w1 x) * (w3 x), fused into the GEMV.
@@ -91,39 +71,13 @@ class DecodeOps:
         Reference: gemv_w4(), kernels/lfm2_decode.cpp:86-98 (batch 1 there; any B >= 1 here). rows is accepted for
         the reference's signature and has no effect. epi (an addition): 0 plain, 1 SwiGLU over Wp = w1|w3
         (R = 2N, y [B, N]), 2 residual add in place into y."""
-        _check_bf16(x, "x")
-        _check_bf16(y, "y")
-        if not (Wp.is_cuda and Wp.is_contiguous() and Wp.dtype == torch.uint8 and Wp.dim() == 2):
-            raise RuntimeError("Wp: contiguous uint8 [N, K/2]")
-        if not (S.is_cuda and S.is_contiguous() and S.dtype == torch.float32):
-            raise RuntimeError("S: contiguous fp32 [N, K/128]")
-        R, K = Wp.size(0), Wp.size(1) * 2
-        group = self._w4_group(S, R, K)
-        B, N = self._w4_shapes(x, y, R, K, epi)
-        _same_device(Wp, S, x, y)
-        _capi.call("lfm2q_gemv_w4", 0, Wp.data_ptr(), S.data_ptr(), None, x.data_ptr(), y.data_ptr(), B, N, K, group,
-                   int(epi), _capi.stream(x))
+        self._n.gemv_w4(Wp, S, x, y, epi)
 
     def gemv_w4z(self, qweight, scales, qzeros, x, y, epi=0):
         """INT4 weight-only GEMV in GPTQ-style storage (an addition): qweight int32 [R, K/8] (nibble i of word w =
         q for k = 8 w + i, q in [0, 15]), scales fp16 [R, K/group], qzeros int32 [R, ceil(K/group/8)] (nibble j of
         word w = zero point of group 8 w + j); w = s (q - z). epi as in gemv_w4."""
-        _check_bf16(x, "x")
-        _check_bf16(y, "y")
-        if not (qweight.is_cuda and qweight.is_contiguous() and qweight.dtype == torch.int32 and qweight.dim() == 2):
-            raise RuntimeError("qweight: contiguous int32 [N, K/8]")
-        if not (scales.is_cuda and scales.is_contiguous() and scales.dtype == torch.float16):
-            raise RuntimeError("scales: contiguous fp16 [N, K/group]")
-        R, K = qweight.size(0), qweight.size(1) * 8
-        group = self._w4_group(scales, R, K)
-        G = K // group
-        if not (qzeros.is_cuda and qzeros.is_contiguous() and qzeros.dtype == torch.int32
-                and tuple(qzeros.shape) == (R, (G + 7) // 8)):
-            raise RuntimeError("qzeros: contiguous int32 [N, ceil(K/group/8)]")
-        B, N = self._w4_shapes(x, y, R, K, epi)
-        _same_device(qweight, scales, qzeros, x, y)
-        _capi.call("lfm2q_gemv_w4", 1, qweight.data_ptr(), scales.data_ptr(), qzeros.data_ptr(), x.data_ptr(),
-                   y.data_ptr(), B, N, K, group, int(epi), _capi.stream(x))
+        self._n.gemv_w4z(qweight, scales, qzeros, x, y, epi)
 
     @staticmethod
     def _w4_group(S, R, K):
@@ -134,26 +88,9 @@ class DecodeOps:
             raise RuntimeError("group size must be a multiple of 32")
         return group
 
-    @staticmethod
-    def _w4_shapes(x, y, R, K, epi):
-        if epi not in (0, 1, 2):
-            raise RuntimeError("epi 0 (none), 1 (swiglu) or 2 (residual)")
-        N = R // 2 if epi == 1 else R
-        B = x.numel() // K if K else 0
-        if not ((epi != 1 or R % 2 == 0) and B >= 1 and x.numel() == B * K and y.numel() == B * N):
-            raise RuntimeError("x [B, K], y [B, N]")
-        return B, N
-
     def silu_mul(self, g, y):
         """y = silu(a) * b on g = [a | b]; reference: silu_mul(), kernels/lfm2_decode.cpp:100-103."""
-        _check_bf16(g, "g")
-        _check_bf16(y, "y")
-        I2 = g.size(-1)
-        B = g.numel() // I2
-        if I2 % 2 or y.numel() != B * (I2 // 2):
-            raise RuntimeError("g [B, 2I], y [B, I]")
-        _same_device(g, y)
-        _capi.call("lfm2q_silu_mul", g.data_ptr(), y.data_ptr(), B, I2 // 2, _capi.stream(g))
+        self._n.silu_mul(g, y)
 
     def gemv_chain(self, ops):
         """A GemvChain over ops [(epi, W, scale, x, y), ...] (an addition): call it to run all of them in one launch."""
@@ -475,29 +412,13 @@ class Int8Ops:
     per-token or grouped-64 activation scales, its INT8-output form gemm_i8_q, and the W8A16 gemm_w8."""
 
     def __init__(self):
-        _capi.lib()
+        self._n = _capi.native()
 
     def gemm_i8(self, xq, sx, w, sw, bias, y, gelu):
         """W8A8: y [M, N] = bf16(gelu?((xq . w^T) * sx[m] * sw[n] + bias[n])), exact int32 accumulation; with 2-D sx
         [K/64, M] (grouped-64 activation scales) the per-group sums fold into fp32 with their scales first.
         Reference: gemm_i8(), kernels/int8_gemm.cpp:39-50."""
-        _check_t(xq, torch.int8, "xq")
-        _check_t(sx, torch.float32, "sx")
-        K = xq.size(-1)
-        M = xq.numel() // K if K else 0
-        grouped = sx.dim() == 2
-        if not ((K % 64 == 0 and sx.size(0) == K // 64 and sx.size(1) == M) if grouped else sx.numel() == M):
-            raise RuntimeError("sx shape")
-        N = self._check_common(w, sw, bias, y, M, K)
-        _same_device(xq, sx, w, sw, bias, y)
-        if grouped:
-            _capi.call("lfm2q_gemm_i8_grouped", xq.data_ptr(), sx.data_ptr(), w.data_ptr(), sw.data_ptr(),
-                       _capi.ptr(bias), y.data_ptr(), M, N, K, int(bool(gelu)), _capi.stream(xq))
-        else:  # per-token: with the stream's workspace (the K split for shapes with fewer tiles than CUs)
-            ws = _capi.workspace(xq)
-            _capi.call("lfm2q_gemm_i8_ex", xq.data_ptr(), sx.data_ptr(), w.data_ptr(), sw.data_ptr(),
-                       _capi.ptr(bias), y.data_ptr(), M, N, K, int(bool(gelu)), ws.data_ptr(), ws.numel(),
-                       _capi.stream(xq))
+        self._n.gemm_i8(xq, sx, w, sw, bias, y, gelu)
 
     def gemm_i8_bf16a(self, x, sx, w, sw, bias, y, gelu):
         """The per-token pair quant_rows(x) + gemm_i8 as one call on bf16 activations x [M, K]: sx [M] receives the
@@ -539,37 +460,12 @@ class Int8Ops:
         """Grouped W8A8 writing the next W8A8 GEMM's input: (yq [M, N], ysT [N/64, M]) = quant_groups(the bf16 output
         gemm_i8 would write), bit-identical to that pair of calls. Reference: gemm_i8_q(), kernels/int8_gemm.cpp:53-69
         (N % 128 there, N % 64 here)."""
-        for t, dt, name in ((xq, torch.int8, "xq"), (sxT, torch.float32, "sxT"), (w, torch.int8, "w"),
-                            (sw, torch.float32, "sw"), (yq, torch.int8, "yq"), (ysT, torch.float32, "ysT")):
-            _check_t(t, dt, name)
-        K = xq.size(-1)
-        M = xq.numel() // K if K else 0
-        N = w.size(0)
-        if not (sxT.dim() == 2 and K % 64 == 0 and sxT.size(0) == K // 64 and sxT.size(1) == M):
-            raise RuntimeError("sxT shape")
-        if not (w.dim() == 2 and w.size(1) == K and N % 64 == 0 and sw.numel() == N):
-            raise RuntimeError("w [N, K] with N % 64 == 0")
-        if not (yq.numel() == M * N and ysT.dim() == 2 and ysT.size(0) == N // 64 and ysT.size(1) == M):
-            raise RuntimeError("yq / ysT shape")
-        if bias is not None:
-            _check_bf16(bias, "bias")
-            if bias.numel() != N:
-                raise RuntimeError("bias shape")
-        _same_device(xq, sxT, w, sw, bias, yq, ysT)
-        _capi.call("lfm2q_gemm_i8_q", xq.data_ptr(), sxT.data_ptr(), w.data_ptr(), sw.data_ptr(), _capi.ptr(bias),
-                   yq.data_ptr(), ysT.data_ptr(), M, N, K, int(bool(gelu)), _capi.stream(xq))
+        self._n.gemm_i8_q(xq, sxT, w, sw, bias, yq, ysT, gelu)
 
     def gemm_w8(self, x, w, sw, bias, y, gelu):
         """W8A16: y [M, N] = bf16(gelu?((x . w^T) * sw[n] + bias[n])), bf16 x, int8 w, fp32 accumulation.
         Reference: gemm_w8(), kernels/int8_gemm.cpp:72-79."""
-        _check_bf16(x, "x")
-        K = x.size(-1)
-        M = x.numel() // K if K else 0
-        N = self._check_common(w, sw, bias, y, M, K)
-        _same_device(x, w, sw, bias, y)
-        ws = _capi.workspace(x)  # the K split across workgroups for shapes with few tiles
-        _capi.call("lfm2q_gemm_w8_ex", x.data_ptr(), w.data_ptr(), sw.data_ptr(), _capi.ptr(bias), y.data_ptr(), M, N,
-                   K, int(bool(gelu)), ws.data_ptr(), ws.numel(), _capi.stream(x))
+        self._n.gemm_w8(x, w, sw, bias, y, gelu)
 
     def gemm_i8_i32(self, xq, w, c):
         """The exact int32 accumulators c [M, N] = xq [M, K] . w [N, K]^T (the torch._int_mm analogue)."""
@@ -592,99 +488,24 @@ class Int8Ops:
         """Symmetric quantization: s = max|x| / 127, q = round(x / s), per row (1-D s [rows]) or per row and group of
         64 columns (2-D s [K/64, rows], transposed as gemm_i8 reads it). Reference: quant_rows(),
         kernels/int8_gemm.cpp:83-96 (K % 128 and, per row, K <= 2048 there; K % 8, grouped K % 64, any K here)."""
-        _check_bf16(x, "x")
-        _check_t(q, torch.int8, "q")
-        _check_t(s, torch.float32, "s")
-        K = x.size(-1)
-        rows = x.numel() // K if K else 0
-        if s.dim() == 2:
-            if not (K % 64 == 0 and K > 0 and s.size(0) == K // 64 and s.size(1) == rows and q.numel() == x.numel()):
-                raise RuntimeError("grouped shapes")
-            _same_device(x, q, s)
-            _capi.call("lfm2q_quant_groups", x.data_ptr(), q.data_ptr(), s.data_ptr(), rows, K, _capi.stream(x))
-            return
-        if K % 8 or K == 0:
-            raise RuntimeError("K must be a multiple of 8")
-        if q.numel() != x.numel() or s.numel() != rows:
-            raise RuntimeError("q / s shape")
-        _same_device(x, q, s)
-        _capi.call("lfm2q_quant_rows", x.data_ptr(), q.data_ptr(), s.data_ptr(), rows, K, _capi.stream(x))
+        self._n.quant_rows(x, q, s)
 
     # ---- fused producers (kernels/int8_gemm.cpp:99-141). x (an addition): also write the bf16 row that was
     # quantized; q / s are then exactly quant_rows(x, ...) of it.
-    @staticmethod
-    def _check_qs(q, s, rows, L):
-        """kernels/int8_gemm.cpp:99-105: per-row (1-D s) or grouped (2-D s [L/64, rows])."""
-        _check_t(q, torch.int8, "q")
-        _check_t(s, torch.float32, "s")
-        grouped = s.dim() == 2
-        if q.numel() != rows * L:
-            raise RuntimeError("q shape")
-        if not (s.size(0) == L // 64 and s.size(1) == rows and L % 64 == 0 if grouped else s.numel() == rows):
-            raise RuntimeError("s shape")
-        return int(grouped)
-
     def add_layernorm_q(self, h, y, w, b, q, s, eps, x=None):
         """vision: h += y (optional, in place, bf16-rounded); (q, s) = quant(LayerNorm(h) * w + b).
         Reference: add_layernorm_q(), kernels/int8_gemm.cpp:108-119 (D % 128, D <= 2048 there; D % 8, D <= 8192)."""
-        _check_bf16(h, "h")
-        _check_bf16(w, "w")
-        _check_bf16(b, "b")
-        if y is not None:
-            _check_bf16(y, "y")
-            if y.numel() != h.numel():
-                raise RuntimeError("y shape")
-        D = h.size(-1)
-        rows = h.numel() // D if D else 0
-        if not (D % 8 == 0 and 0 < D <= 8192 and w.numel() == D and b.numel() == D):
-            raise RuntimeError("D must be a multiple of 8, <= 8192")
-        grouped = self._check_qs(q, s, rows, D)
-        if x is not None:
-            _check_bf16(x, "x")
-            if x.numel() != h.numel():
-                raise RuntimeError("x shape")
-        _same_device(h, y, w, b, q, s, x)
-        _capi.call("lfm2q_add_layernorm_q", h.data_ptr(), _capi.ptr(y), w.data_ptr(), b.data_ptr(), q.data_ptr(),
-                   s.data_ptr(), _capi.ptr(x), rows, D, float(eps), grouped, _capi.stream(h))
+        self._n.add_layernorm_q(h, y, w, b, q, s, eps, x)
 
     def add_rmsnorm_q(self, h, y, w, q, s, eps, x=None):
         """LM prefill: h += y (optional, in place, bf16-rounded); (q, s) = quant(bf16(w * bf16(rmsnorm(h)))).
         Reference: add_rmsnorm_q(), kernels/int8_gemm.cpp:122-132 (H <= 8192 here)."""
-        _check_bf16(h, "h")
-        _check_bf16(w, "w")
-        if y is not None:
-            _check_bf16(y, "y")
-            if y.numel() != h.numel():
-                raise RuntimeError("y shape")
-        H = h.size(-1)
-        rows = h.numel() // H if H else 0
-        if not (w.numel() == H and H % 8 == 0 and 0 < H <= 8192):
-            raise RuntimeError("w shape")
-        grouped = self._check_qs(q, s, rows, H)
-        if x is not None:
-            _check_bf16(x, "x")
-            if x.numel() != h.numel():
-                raise RuntimeError("x shape")
-        _same_device(h, y, w, q, s, x)
-        _capi.call("lfm2q_add_rmsnorm_q", h.data_ptr(), _capi.ptr(y), w.data_ptr(), q.data_ptr(), s.data_ptr(),
-                   _capi.ptr(x), rows, H, float(eps), grouped, _capi.stream(h))
+        self._n.add_rmsnorm_q(h, y, w, q, s, eps, x)
 
     def silu_mul_q(self, g, q, s, x=None):
         """LM prefill: g [rows, 2I] = w1 | w3 outputs -> (q, s) = quant(bf16(bf16(silu(g1)) * g3)).
         Reference: silu_mul_q(), kernels/int8_gemm.cpp:135-141 (I % 64, I <= 20000 there; I % 8, I <= 8192)."""
-        _check_bf16(g, "g")
-        I = g.size(-1) // 2
-        rows = g.numel() // (2 * I) if I else 0
-        if not (I % 8 == 0 and 0 < I <= 8192 and g.size(-1) == 2 * I):
-            raise RuntimeError("I shape")
-        grouped = self._check_qs(q, s, rows, I)
-        if x is not None:
-            _check_bf16(x, "x")
-            if x.numel() != rows * I:
-                raise RuntimeError("x shape")
-        _same_device(g, q, s, x)
-        _capi.call("lfm2q_silu_mul_q", g.data_ptr(), q.data_ptr(), s.data_ptr(), _capi.ptr(x), rows, I, grouped,
-                   _capi.stream(g))
+        self._n.silu_mul_q(g, q, s, x)
 
     @staticmethod
     def _check_common(w, sw, bias, y, M, K):
