@@ -64,6 +64,13 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(lane_read(v, 0), lane_read(v, 16)), fmaxf(lane_read(v, 32), lane_read(v, 48)));
 }
 
+// Maximum over 8 consecutive lanes (a 64-column group of 8-value vectors); every lane receives it. Values >= 0.
+__device__ __forceinline__ float max8(float v) {
+    v = fmaxf(v, dpp<DPP_XOR1>(v));
+    v = fmaxf(v, dpp<DPP_XOR2>(v));
+    return fmaxf(v, dpp<DPP_HALF_MIRROR>(v));
+}
+
 // Sums of V values (V = 1, 2, 4, 8) over the 64 lanes of a wavefront in one transposed reduction: lane bits 5, 4
 // and 3 are folded first -- while several values remain, each fold pairs two of them, so that half the lanes add
 // the partner's copy of one value and the other half of the other (permlane32 / permlane16 swaps, then a DPP row
@@ -197,6 +204,35 @@ __device__ __forceinline__ float silu_f32(float g) {
     const float rr = __builtin_fmaf(q, __builtin_fminf(ds, 0x1p64f), -gs);
     const float res = __builtin_fmaf(-rr, r, q);
     return g == __builtin_inff() ? g : res;
+}
+
+// bf16(silu) of 8 bf16 values (one 16-byte vector), as fp32: silu_f32's bits after the rounding at a third of its
+// instructions. For |g| < 32 neither the clamp, the scaling nor the compensation of the exponent's argument matters to the
+// rounded result (equal to silu_f32's for every bf16 of that range); a vector with a larger value or a NaN takes silu_f32.
+// silu_mul_q, bound by its vector operations, with this and max8 in place of LDS permutes, 8192 wide on MI355X: 4096 rows
+// 47.6 -> 37.8 us, 2048 27.9 -> 21.6, 461 10.8 -> 8.7.
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void silu8_bf16(v4i gv, float (&o)[8]) {
+#pragma clang fp contract(off)
+    float g[8];
+    v2us m = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        g[2 * j] = bf2f_lo((uint32_t)gv[j]);
+        g[2 * j + 1] = bf2f_hi((uint32_t)gv[j]);
+        m = __builtin_elementwise_max(m, __builtin_bit_cast(v2us, gv[j] & 0x7fff7fff));
+    }
+    if (__builtin_expect(max((int)m[0], (int)m[1]) >= 0x4200, 0)) {  // |g| >= 32, inf or NaN
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = rbf(silu_f32(g[e]));
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float d = 1.f + __builtin_amdgcn_exp2f(-g[e] * 1.44269502f);
+            const float r = __builtin_amdgcn_rcpf(d), q = g[e] * r;
+            o[e] = rbf(__builtin_fmaf(-__builtin_fmaf(q, d, -g[e]), r, q));
+        }
+    }
 }
 
 // GELU, tanh form: 0.5 v (1 + tanh(u)), u = sqrt(2/pi) (v + 0.044715 v^3), with 1 + tanh(u) formed in fp32 as the

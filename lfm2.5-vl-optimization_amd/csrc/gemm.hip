@@ -247,11 +247,7 @@ __device__ __forceinline__ void store_tile_staged(const ACC (&acc)[TN][TM], cons
                 // the 8 lanes c0 .. c0 + 7 (c0 % 8 == 0) of this row hold one 64-column group of bf16 outputs:
                 // quantize it exactly as quant_groups does
                 const v4i xv = v4i{(int)v0.x, (int)v0.y, (int)v1.x, (int)v1.y};
-                float am = absmax8(xv, 0.f);
-                am = fmaxf(am, __shfl_xor(am, 1));
-                am = fmaxf(am, __shfl_xor(am, 2));
-                am = fmaxf(am, __shfl_xor(am, 4));
-                const float sc = scale_of(am);
+                const float sc = scale_of(max8(absmax8(xv, 0.f)));
                 if (mo < M && no < N) {
                     int lo, hi;
                     quant8(xv, sc, 1.f / sc, lo, hi);

@@ -16,12 +16,6 @@ namespace {
 constexpr int HD = 64;         // head_dim
 constexpr int DPP_XOR3 = 0x1b;  // quad_perm [3, 2, 1, 0]
 
-__device__ __forceinline__ float max8(float v) {  // over 8 consecutive lanes
-    v = fmaxf(v, dpp<DPP_XOR1>(v));
-    v = fmaxf(v, dpp<DPP_XOR2>(v));
-    return fmaxf(v, dpp<DPP_HALF_MIRROR>(v));
-}
-
 // ------------------------------------------------------------------------------------------------ q / k / v
 // One workgroup per (32 positions, kv head, batch row): thread t holds dims 8 (t % 8) .. + 7 of position t / 8, so a head
 // is 8 lanes (the squares' sum and the rotary partner, dims + 32, are DPP permutations). The group's q heads and the k head

@@ -42,11 +42,7 @@ __device__ __forceinline__ void quant_store(const v4i (&v)[CH], int C, int8_t *_
         const int i = c * 64 + lane;
         float sc = sc_row, rc = rc_row;
         if (GROUPED) {
-            float m = absmax8(v[c], 0.f);
-            m = fmaxf(m, __shfl_xor(m, 1));
-            m = fmaxf(m, __shfl_xor(m, 2));
-            m = fmaxf(m, __shfl_xor(m, 4));
-            sc = scale_of(m);
+            sc = scale_of(max8(absmax8(v[c], 0.f)));
             rc = 1.f / sc;
             if (i < C && (lane & 7) == 0) s[(size_t)(i >> 3) * rows + row] = sc;
         }
@@ -131,11 +127,7 @@ __device__ __forceinline__ void quant_store_wg(const v4i (&v)[CH], int C, int8_t
         const int i = c * 256 + t;
         float sc = sc_row, rc = rc_row;
         if (GROUPED) {
-            float m = absmax8(v[c], 0.f);
-            m = fmaxf(m, __shfl_xor(m, 1));
-            m = fmaxf(m, __shfl_xor(m, 2));
-            m = fmaxf(m, __shfl_xor(m, 4));
-            sc = scale_of(m);
+            sc = scale_of(max8(absmax8(v[c], 0.f)));
             rc = 1.f / sc;
             if (i < C && (t & 7) == 0) s[(size_t)(i >> 3) * rows + row] = sc;
         }
@@ -401,10 +393,11 @@ __global__ __launch_bounds__(256) void silu_mul_q_kernel(const uint16_t *__restr
         xv[c] = v4i{0, 0, 0, 0};
         if (i < C) {
             const v4i av = ld_nt16(gr + (size_t)i * 8), uv = ld_nt16(gr + I + (size_t)i * 8);
+            float sv[8];
+            silu8_bf16(av, sv);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                xv[c][j] = (int)pack_bf16x2(rbf(silu_f32(bf2f_lo((uint32_t)av[j]))) * bf2f_lo((uint32_t)uv[j]),
-                                      rbf(silu_f32(bf2f_hi((uint32_t)av[j]))) * bf2f_hi((uint32_t)uv[j]));
+                xv[c][j] = (int)pack_bf16x2(sv[2 * j] * bf2f_lo((uint32_t)uv[j]), sv[2 * j + 1] * bf2f_hi((uint32_t)uv[j]));
         }
     }
     if (xo) store_row<CH>(xo + (size_t)row * I, xv, C, lane);
@@ -438,10 +431,11 @@ __global__ __launch_bounds__(256) void silu_mul_q_wg_kernel(const uint16_t *__re
         const int i = c * 256 + t;
         xv[c] = v4i{0, 0, 0, 0};
         if (i < C) {
+            float sv[8];
+            silu8_bf16(av[c], sv);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                xv[c][j] = (int)pack_bf16x2(rbf(silu_f32(bf2f_lo((uint32_t)av[c][j]))) * bf2f_lo((uint32_t)uv[c][j]),
-                                      rbf(silu_f32(bf2f_hi((uint32_t)av[c][j]))) * bf2f_hi((uint32_t)uv[c][j]));
+                xv[c][j] = (int)pack_bf16x2(sv[2 * j] * bf2f_lo((uint32_t)uv[c][j]), sv[2 * j + 1] * bf2f_hi((uint32_t)uv[c][j]));
             if (xo) *reinterpret_cast<v4i *>(xo + (size_t)row * I + (size_t)i * 8) = xv[c];
         }
     }
@@ -558,7 +552,7 @@ extern "C" int lfm2q_add_rmsnorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm
     }
 #define LFM2Q_P(CH_)                                                                                                 \
     if (grouped)                                                                                                     \
-        add_rmsnorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, q, s, x, rows, H, eps);                       \
+        add_rmsnorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, q, s, x, rows, H, eps);                    \
     else                                                                                                             \
         add_rmsnorm_q_kernel<CH_, false><<<grid, 256, 0, st>>>(h, y, w, q, s, x, rows, H, eps)
     LFM2Q_CH_SWITCH(H, LFM2Q_P)
@@ -578,7 +572,7 @@ extern "C" int lfm2q_add_layernorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const l
     const hipStream_t st = (hipStream_t)stream;
 #define LFM2Q_P(CH_)                                                                                                 \
     if (grouped)                                                                                                     \
-        add_layernorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, b, q, s, x, rows, D, eps);                  \
+        add_layernorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, b, q, s, x, rows, D, eps);             \
     else                                                                                                             \
         add_layernorm_q_kernel<CH_, false><<<grid, 256, 0, st>>>(h, y, w, b, q, s, x, rows, D, eps)
     LFM2Q_CH_SWITCH(D, LFM2Q_P)
