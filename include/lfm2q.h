@@ -195,6 +195,18 @@ size_t lfm2q_attn_step_workspace_bytes(int B, int n_heads, int n_kv, int max_len
 int lfm2q_conv_step(const lfm2q_bf16 *bcx, lfm2q_bf16 *ring, const lfm2q_bf16 *wt, const lfm2q_bf16 *bias,
                     const int64_t *ctr, lfm2q_bf16 *out, int B, int H, int L, lfm2q_stream_t stream);
 
+/* The batch-1 projection of a short-conv layer and its conv step in one launch: bcx [1, 3 H] = the GEMV of RMSNorm(h) over
+ * W = b | c | x [3 H, K] (as lfm2q_gemv_rmsnorm / lfm2q_gemv_w4_rmsnorm with epi 0), then lfm2q_conv_step of it (B = 1);
+ * bit-identical to that pair. L = 3. K in {1024, 2048, 4096} for INT8, {512, 1024, 2048} for bf16, 128 .. 2048 for INT4.
+ * Replaces gemv_epi(1, ...) kernels/lfm2_decode.cu:724-805 with the norm before it. */
+int lfm2q_gemv_conv_rmsnorm(int wtype, const void *W, const float *scale, const lfm2q_bf16 *h, const lfm2q_bf16 *norm_w,
+                            float eps, lfm2q_bf16 *ring, const lfm2q_bf16 *wt, const lfm2q_bf16 *bias, const int64_t *ctr,
+                            lfm2q_bf16 *out, int H, int K, int L, lfm2q_stream_t stream);
+int lfm2q_gemv_w4_conv_rmsnorm(int fmt, const void *Wq, const void *S, const int32_t *Z, const lfm2q_bf16 *h,
+                               const lfm2q_bf16 *norm_w, float eps, lfm2q_bf16 *ring, const lfm2q_bf16 *wt,
+                               const lfm2q_bf16 *bias, const int64_t *ctr, lfm2q_bf16 *out, int H, int K, int group, int L,
+                               lfm2q_stream_t stream);
+
 /* h bf16 [B, H] = the rows tok[b] of table bf16 [V, H] (NaN for a token outside it). H % 8 == 0, table and h 16-byte
  * aligned. Replaces the embedding lookup of the reference's step (src/lfm2opt/runtime.py:246-250). */
 int lfm2q_embed_step(const lfm2q_bf16 *table, const int64_t *tok, lfm2q_bf16 *h, int B, int H, int V,

@@ -40,6 +40,8 @@ SIGNATURES = {
     "lfm2q_gemv_rmsnorm": [_I, _I, _P, _P, _P, _P, _F, _P, _I, _I, _P],
     "lfm2q_gemv_w4": [_I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P],
     "lfm2q_gemv_w4_rmsnorm": [_I, _P, _P, _P, _P, _P, _F, _P, _I, _I, _I, _I, _P],
+    "lfm2q_gemv_conv_rmsnorm": [_I, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _I, _P],
+    "lfm2q_gemv_w4_conv_rmsnorm": [_I, _P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P],
     "lfm2q_add_rmsnorm": [_P, _P, _P, _P, _I, _I, _F, _P],
     "lfm2q_attn_step": [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _F, _P, ctypes.c_size_t, _P],
     "lfm2q_attn_step_workspace_bytes": [_I, _I, _I, _I],

@@ -239,6 +239,13 @@ class DecodeLinears:
         self.K.gemv_rmsnorm(w, self.lin_scale.get(key), h.contiguous(), norm_w, eps, y, 1 if swiglu else 0)
         return y
 
+    def conv_normed(self, h, key, norm_w, eps, ring, wt, bias, ctr, out):
+        """The projection under key of rms_norm(h) * norm_w and the short-conv step of it into out, as one GEMV
+        (norm_fusable(1, key) and K <= 2048 must hold, ring [3, 1, H]): bit-identical to linear_normed, then conv_step."""
+        self.last_path = "gemv"
+        self.K.gemv_conv_rmsnorm(self.lin[key], self.lin_scale.get(key), self.lin_zeros.get(key), h.contiguous(), norm_w,
+                                 eps, ring, wt, bias, ctr, out)
+
     def residual(self, x, key, h):
         """h [B, N] = bf16(h + bf16(x @ W^T)) in place: the GEMV's fused residual epilogue on the GEMV path, else the
         linear and a BF16 add (the rounding of the residual add in the reference's add_rmsnorm)."""

@@ -162,6 +162,50 @@ class DecodeOps:
         _capi.call("lfm2q_gemv_w4_rmsnorm", fmt, Wp.data_ptr(), S.data_ptr(), _capi.ptr(zeros), h.data_ptr(),
                    norm_w.data_ptr(), float(eps), y.data_ptr(), N, K, group, int(epi), _capi.stream(h))
 
+    def gemv_conv_rmsnorm(self, W, scale, zeros, h, norm_w, eps, ring, wt, bias, ctr, out):
+        """The batch-1 projection of a short-conv layer and its conv step in one launch (an addition): the GEMV of
+        RMSNorm(h) over W = b | c | x [3 H, K] (INT8 or bf16 with its scale, or INT4 as in gemv_w4_rmsnorm), then conv_step
+        of it with ring [3, 1, H]; bit-identical to that pair. Replaces gemv_epi(1, ...), kernels/lfm2_decode.cpp:130-150,
+        with the norm before it."""
+        for t, name in ((h, "h"), (norm_w, "norm_w"), (ring, "ring"), (wt, "wt"), (out, "out")):
+            _check_bf16(t, name)
+        _check_t(ctr, torch.int64, "ctr")
+        if bias is not None:
+            _check_bf16(bias, "bias")
+        if not (W.is_cuda and W.is_contiguous() and W.dim() == 2 and ring.dim() == 3):
+            raise RuntimeError("gemv_conv_rmsnorm: W [3 H, K] contiguous, ring [L, 1, H]")
+        per = {torch.int8: 1, torch.bfloat16: 1, torch.uint8: 2, torch.int32: 8}.get(W.dtype)
+        if per is None:
+            raise RuntimeError("W must be int8, bf16, uint8 (INT4) or int32 (INT4)")
+        R, K = W.size(0), W.size(1) * per
+        L, B, H = ring.shape
+        if not (R == 3 * H and B == 1 and h.numel() == K and norm_w.numel() == K and tuple(wt.shape) == (L, H)
+                and out.numel() == H and ctr.numel() >= 1 and (bias is None or bias.numel() == H)):
+            raise RuntimeError("gemv_conv_rmsnorm: W [3 H, K], h [1, K], ring [L, 1, H], wt [L, H], out [1, H] (batch 1)")
+        tail = (h.data_ptr(), norm_w.data_ptr(), float(eps), ring.data_ptr(), wt.data_ptr(), _capi.ptr(bias),
+                ctr.data_ptr(), out.data_ptr(), H, K)
+        if per == 1:
+            if W.dtype == torch.int8 and scale is None:
+                raise RuntimeError("int8 W needs fp32 scale")
+            if scale is not None:
+                _check_t(scale, torch.float32, "scale")
+                if scale.numel() != R:
+                    raise RuntimeError("scale must have one value per weight row")
+            _same_device(W, scale, h, norm_w, ring, wt, bias, ctr, out)
+            _capi.call("lfm2q_gemv_conv_rmsnorm", 0 if W.dtype == torch.int8 else 1, W.data_ptr(), _capi.ptr(scale), *tail,
+                       L, _capi.stream(h))
+            return
+        fmt = 0 if per == 2 else 1
+        _check_t(scale, torch.float32 if fmt == 0 else torch.float16, "S")
+        group = self._w4_group(scale, R, K)
+        if fmt == 1:
+            _check_t(zeros, torch.int32, "zeros")
+            if tuple(zeros.shape) != (R, (K // group + 7) // 8):
+                raise RuntimeError("qzeros: contiguous int32 [N, ceil(K/group/8)]")
+        _same_device(W, scale, zeros, h, norm_w, ring, wt, bias, ctr, out)
+        _capi.call("lfm2q_gemv_w4_conv_rmsnorm", fmt, W.data_ptr(), scale.data_ptr(), _capi.ptr(zeros), *tail, group, L,
+                   _capi.stream(h))
+
     def add_rmsnorm(self, h, y, w, x, eps):
         """h += y (optional, in place, bf16-rounded); x = bf16(w * bf16(rmsnorm(h))): add_rmsnorm_q's h and x without the
         INT8 row. Reference: add_rmsnorm(), kernels/lfm2_decode.cpp:33-38."""

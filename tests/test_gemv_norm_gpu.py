@@ -193,3 +193,48 @@ def test_gemv_w4_rmsnorm_equals_norm_then_gemv(E, E8, fmt, R, epi, K, group, tun
         E.gemv_w4z(W, S, Z, x, ref, epi=epi)
     E.gemv_w4_rmsnorm(W, S, Z, h, nw, 1e-5, y, epi)
     assert np.array_equal(host_bits(y), host_bits(ref))
+
+
+@pytest.mark.parametrize("wt,K", [("int8", 1024), ("int8", 2048), ("int8", 4096), ("bf16", 512), ("bf16", 2048),
+                                  ("w4", 2048), ("w4", 128), ("w4z", 1120), ("w4z", 2048)])
+@pytest.mark.parametrize("H,bias", [(1, False), (7, True), (2048, False)])
+def test_gemv_conv_rmsnorm_equals_the_pair(E, wt, K, H, bias):
+    """Outputs and ring bit for bit those of the normalizing GEMV, then conv_step, over five positions of a ring (each
+    slot, negative products and the ring's own earlier rows)."""
+    g = torch.Generator().manual_seed(H + K)
+    R, Z = 3 * H, None
+    if wt == "int8" or wt == "bf16":
+        W, S = weights(g, R, K, wt == "int8")
+    elif wt == "w4":
+        W = torch.randint(0, 256, (R, K // 2), generator=g, dtype=torch.uint8).cuda()
+        S = (torch.rand(R, K // 32, generator=g) * 0.01).cuda()
+    else:
+        G = K // 32
+        W = torch.randint(-2**31, 2**31 - 1, (R, K // 8), generator=g, dtype=torch.int64).to(torch.int32).cuda()
+        S = (torch.rand(R, G, generator=g) * 0.01).half().cuda()
+        Z = torch.randint(0, 2**31 - 1, (R, (G + 7) // 8), generator=g, dtype=torch.int64).to(torch.int32).cuda()
+    nw = (torch.rand(K, generator=g) + 0.5).to(torch.bfloat16).cuda()
+    taps = torch.randn(3, H, generator=g).to(torch.bfloat16).cuda()
+    b = torch.randn(H, generator=g).to(torch.bfloat16).cuda() if bias else None
+    ring = torch.randn(3, 1, H, generator=g).to(torch.bfloat16).cuda()
+    ref_ring = ring.clone()
+    pad = -H % 4  # conv_step takes channels in fours
+    for pos in range(4, 9):
+        h, ctr = row(g, K), torch.tensor([pos, 0], device="cuda")
+        out = torch.empty(1, H, device="cuda", dtype=torch.bfloat16)
+        E.gemv_conv_rmsnorm(W, S, Z, h, nw, 1e-5, ring, taps, b, ctr, out)
+        bcx = torch.empty(1, R, device="cuda", dtype=torch.bfloat16)
+        if wt == "int8" or wt == "bf16":
+            E.gemv_rmsnorm(W, S, h, nw, 1e-5, bcx, 0)
+        else:
+            E.gemv_w4_rmsnorm(W, S, Z, h, nw, 1e-5, bcx, 0)
+
+        def wide(t):
+            return torch.nn.functional.pad(t, (0, pad)).contiguous()
+
+        want, rr = torch.empty(1, H + pad, device="cuda", dtype=torch.bfloat16), wide(ref_ring)
+        E.conv_step(torch.cat([wide(t) for t in bcx.chunk(3, -1)], -1), rr, wide(taps), None if b is None else wide(b), ctr,
+                    want)
+        ref_ring = rr[..., :H].contiguous()
+        assert np.array_equal(host_bits(out), host_bits(want[:, :H].contiguous())), f"position {pos}"
+        assert torch.equal(ring, ref_ring)
