@@ -178,7 +178,7 @@ int lfm2q_silu_mul(const lfm2q_bf16 *g, lfm2q_bf16 *y, int B, int I, lfm2q_strea
  * fp32 [max_len, 2, head_dim]: cos and sin per position; k bf16 [B, n_kv, head_dim, max_len] (keys transposed), v bf16
  * [B, n_kv, max_len, head_dim]. head_dim 64, n_heads / n_kv in {1, 2, 4, 8}, max_len % 8 == 0; qkv, k, v 16-byte
  * aligned. ws: lfm2q_attn_step_workspace_bytes() of device memory (may be 0), contents irrelevant, not shared by
- * overlapping calls. A position outside the cache is a device trap.
+ * overlapping calls. A position outside the cache gives NaN in out.
  * Replaces the reference step's q / k norm, rotary embedding, cache write and attention (src/lfm2opt/runtime.py:
  * 256-271). */
 int lfm2q_attn_step(const lfm2q_bf16 *qkv, const float *qk_w, const float *rope, const int64_t *ctr, lfm2q_bf16 *k,

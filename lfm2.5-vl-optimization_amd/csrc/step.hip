@@ -29,11 +29,10 @@ namespace {
 constexpr int HD = 64;   // head_dim
 constexpr int PC = 256;  // cache positions per chunk
 
-// The step's cache position. One outside the cache ends the program, as an out-of-range index of a tensor op does.
+// The step's cache position, -1 outside the cache (its output is NaN then, and nothing else is read or written).
 __device__ __forceinline__ int cache_pos(const int64_t *__restrict__ ctr, int max_len) {
     const int64_t p = ctr[0];
-    if (p < 0 || p >= max_len) __builtin_trap();
-    return (int)p;
+    return p < 0 || p >= max_len ? -1 : (int)p;
 }
 
 // head row `row` (q heads, then k heads) of the projection, normalized and rotated; lane d holds dim d. qkw: the head
@@ -60,6 +59,11 @@ __global__ __launch_bounds__(256) void attn_step_kernel(const uint16_t *__restri
     const int h0 = kv * grp + (blockIdx.y / nkv) * G;  // this workgroup's first query head
     const int nh = nkv * grp, ld = (nh + 2 * nkv) * HD;
     const int pos = cache_pos(ctr, max_len);
+    if (pos < 0) {
+        if (split == 0)
+            for (int i = t; i < G * HD; i += 256) out[((size_t)b * nh + h0) * HD + i] = 0x7fff;
+        return;
+    }
     int p0 = split * chunks * PC;
     if (p0 > pos) return;  // uniform; the combine pass skips this split as well
     const int last = min(pos, p0 + chunks * PC - 1);  // this workgroup's last position
@@ -233,6 +237,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float *__restri
     const int row = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));  // (batch row, head)
     if (row >= heads) return;
     const int pos = cache_pos(ctr, max_len);
+    if (pos < 0) return;  // attn_step_kernel has written NaN
     const int n = pos / (chunks * PC) + 1;  // splits that hold positions
     const float *pp = part + (size_t)row * splits * (HD + 2);
     // lane i takes split i's maximum and sum (splits <= 64); the first 16 splits' outputs are in flight with them

@@ -65,6 +65,18 @@ def test_attn_step(cuda, G, B, max_len, positions):
         assert kc[..., pos + 1:].isnan().all() and vc[:, :, pos + 1:].isnan().all()
 
 
+@pytest.mark.parametrize("pos,max_len", [(-1, 64), (64, 64), (4096, 4096)])
+def test_attn_step_outside_the_cache(cuda, pos, max_len):
+    """A position outside the cache gives NaN and leaves the cache alone (one chunk, and several splits)."""
+    from lfm2opt.kernels import ext
+
+    E, z = ext(), lambda *s, dt=torch.bfloat16: torch.zeros(*s, dtype=dt, device=cuda)  # noqa: E731
+    k, v, out = z(2, 2, 64, max_len), z(2, 2, max_len, 64), z(2, 4 * 64)
+    E.attn_step(z(2, 8 * 64) + 1, z(2, 6, 64, dt=torch.float32), z(max_len, 2, 64, dt=torch.float32),
+                torch.tensor([pos, 0], device=cuda), k, v, out, 0.1, 1e-5, E.attn_step_workspace(2, 4, 2, max_len, cuda))
+    assert out.isnan().all() and not k.any() and not v.any()
+
+
 def test_attn_step_refuses_other_shapes(cuda):
     from lfm2opt.kernels import ext
 
