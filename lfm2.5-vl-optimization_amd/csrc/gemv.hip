@@ -41,12 +41,12 @@ namespace {
 // i.e. vectors XL (l + 64 u) + q. NORM: x is the RMSNorm of the row h with weight nw, computed here exactly as
 // add_rmsnorm_q computes it (rmsnorm.hpp), so the GEMV of the normalized row equals add_rmsnorm_q followed by the
 // GEMV bit for bit: the sum of squares is taken in add_rmsnorm_q's order -- lane l sums vectors c 64 + l, c < CH =
-// CPL XL -- by fetching those vectors from the lanes that hold them (for XL = 2 vector c 64 + l is register
-// [c / 2][l % 2] of lane 32 (c % 2) + l / 2; for XL = 1 the two layouts coincide), then x = bf16(w bf16(h rs))
+// CPL XL -- by loading those vectors as well (they are in the L1 with the lane's own; fetching them from the lanes that
+// hold them took 8 LDS permutes a vector; for XL = 1 the two layouts coincide), then x = bf16(w bf16(h rs))
 // elementwise in the kernel's own layout. Needs K = 64 PER CPL exactly (every vector in range).
 template <int PER, int XL, int CPL, bool NORM>
 struct XLoadB1 {
-    v4i hv[CPL][XL], wv[CPL][XL];
+    v4i hv[CPL][XL], wv[CPL][XL], sv[XL == 1 ? 1 : CPL * XL];
     // NORM: the row and the norm weight, in flight before the caller issues its weight loads
     __device__ __forceinline__ void issue(const uint16_t *__restrict__ x, const uint16_t *__restrict__ nw, int lane) {
         if constexpr (NORM) {
@@ -57,6 +57,9 @@ struct XLoadB1 {
                     hv[u][q] = ld16(x + (size_t)(lane + 64 * u) * PER + 8 * q);
                     wv[u][q] = ld16(nw + (size_t)(lane + 64 * u) * PER + 8 * q);
                 }
+            if constexpr (XL > 1)
+#pragma unroll
+                for (int c = 0; c < CPL * XL; ++c) sv[c] = ld16(x + (size_t)(c * 64 + lane) * 8);
         }
     }
     __device__ __forceinline__ void finish(const uint16_t *__restrict__ x, float eps, int K, int lane,
@@ -69,20 +72,7 @@ struct XLoadB1 {
         } else {
             float ss = 0.f;
 #pragma unroll
-            for (int c = 0; c < CPL * XL; ++c) {
-                if constexpr (XL == 1) {
-                    ss = sumsq8(hv[c][0], ss);
-                } else {
-                    const int src = 32 * (c & 1) + (lane >> 1);
-                    v4i g;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int a = __shfl(hv[c >> 1][0][j], src), b = __shfl(hv[c >> 1][1][j], src);
-                        g[j] = (lane & 1) ? b : a;
-                    }
-                    ss = sumsq8(g, ss);
-                }
-            }
+            for (int c = 0; c < CPL * XL; ++c) ss = sumsq8(XL == 1 ? hv[c][0] : sv[c], ss);
             const float rs = rms_scale(wave_sum(ss), K, eps);
 #pragma unroll
             for (int u = 0; u < CPL; ++u)

@@ -699,9 +699,10 @@ void launch_w4_b1(const uint8_t *W, const void *S, const int32_t *Z, const uint1
         // graph of that kind alone (w1|w3 5.41 -> 5.17 us, o/out_proj 3.83 -> 3.71, w2 4.62 -> 4.50, qkv 3.79 ->
         // 3.71), but in the 65-kernel decode step it on qkv / in_proj or on w2 lengthened the step by ~2.5 us while
         // shortening the kernels (a kernel trace shows the time moving into the gaps between kernels; not
-        // understood), and on w1|w3 or o/out_proj alone it is neutral to -0.4 us
+        // understood), and on w1|w3 or o/out_proj alone it is neutral to -0.4 us. The normalizing form always takes it
+        // (one wavefront of four normalizes and repacks: three-layer steps 745 -> 736 us for eight)
         const int xs_forced = knob_int(KNOB_GEMV_XS, -1);
-        const bool xs = xs_forced >= 0 ? xs_forced == 1 : EPI == EPI_SWIGLU || (EPI == EPI_RESIDUAL && C <= 64);
+        const bool xs = xs_forced >= 0 ? xs_forced == 1 : NORM || EPI == EPI_SWIGLU || (EPI == EPI_RESIDUAL && C <= 64);
 #define LFM2Q_W4O(C_)                                                                                 \
     do {                                                                                              \
         if (xs)                                                                                       \
