@@ -4,7 +4,9 @@
 src/lfm2opt/kernels.py:16-32,66-68. The ops keep their names, argument order and meaning, destination-passing
 style (every output is preallocated by the caller, ops return None) and launch on torch's current stream. Argument
 errors raise RuntimeError with the reference's TORCH_CHECK wording (kernels/lfm2_decode.cpp:28-150) before any
-launch. Ops outside the quantized-matmul path (attention, norms, convolutions) are not provided.
+launch. The reference's attention and convolution ops are not provided under its names; the decode step's and the prompt
+pass's have kernels of their own (attn_step, conv_step, prompt_attn, ...). The hot ops' checks and calls are native
+(_capi.native()).
 """
 
 import ctypes
