@@ -102,8 +102,8 @@ __global__ __launch_bounds__(256) void prompt_qkv_kernel(uint16_t *qkv, const fl
 // the row maximum, its correction and the sum stay in the lane, and the probabilities, rounded to bf16, are the next
 // product's operand (O^T = V^T P^T) in the registers they are in: vt's order of positions is the lanes'. Bound by the
 // softmax's VALU work (an exponential costs 16 cycles a wavefront; 64 dims give each only two short products). MI355X, 32
-// heads over 8: 16.0 us at 461 positions and 53.4 at 2,048; the PyTorch ops they replace (masked products, softmax, copies)
-// and the launches of prompt_qkv took about 150 and 390.
+// heads over 8: 16.0 us at 461 positions and 53.4 at 2,048; the PyTorch ops that this kernel and prompt_qkv replace (norm,
+// rotary embedding, masked products, softmax, copies) took about 120 and 560.
 template <int GW, bool QUANT>
 __global__ __launch_bounds__(256) void prompt_attn_kernel(const uint16_t *__restrict__ qkv,
                                                           const uint16_t *__restrict__ vt, uint16_t *__restrict__ out,
@@ -266,8 +266,8 @@ __global__ __launch_bounds__(256) void prompt_attn_kernel(const uint16_t *__rest
 // c | x; with u = b x rounded, y = sum over the taps of rounded products (fp32, newest last as the decode step's taps), the
 // bias, times c, each rounded as the bf16 tensor ops round. The last L positions' u become the ring's rows (position p in
 // row p mod L; rows of positions before the prompt zero). Bound by memory: 4 H values in and out a position. MI355X,
-// 2,048 channels, with the quantized output: 7.8 us at 461 positions and 12.0 at 2,048, in place of twelve PyTorch launches
-// (~35 and ~100 us) and the quantizer.
+// 2,048 channels, with the quantized output: 7.8 us at 461 positions and 12.0 at 2,048, in place of ten PyTorch launches
+// (41 and 59 us) and the quantizer (3.7 and 5.6).
 constexpr int CP = 4;
 
 template <int L, bool QUANT>
