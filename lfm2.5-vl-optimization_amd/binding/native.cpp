@@ -83,43 +83,50 @@ float real(PyObject *o) {
     return (float)v;
 }
 
-// a library call without the interpreter lock; a non-zero status becomes RuntimeError with the library's message
-template <typename F>
-void run(F &&f) {
-    int st;
-    Py_BEGIN_ALLOW_THREADS;
-    st = f();
-    Py_END_ALLOW_THREADS;
-    if (st != LFM2Q_OK) fail(lfm2q_last_error());
+// The interpreter lock released for a scope, and taken again however the scope is left
+class Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+
+  public:
+    Unlocked() = default;
+    Unlocked(const Unlocked &) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// The library call f(a..., the current stream of on's device) without the interpreter lock; a non-zero status becomes
+// RuntimeError with the library's message. The arguments, pointers among them, are values by now: reading the pointer of
+// a tensor that has none (a vmap wrapper) throws, and must do so while the lock is held.
+template <typename... P, typename... A>
+void run(const Tensor &on, int (*f)(P...), A... a) {
+    const lfm2q_stream_t st = stream(on);
+    int status;
+    {
+        const Unlocked unlocked;
+        status = f(a..., st);
+    }
+    if (status != LFM2Q_OK) fail(lfm2q_last_error());
 }
 
 // The GEMM workspace of t's device and current stream: the entry of lfm2opt._capi's table, made by its prepare_workspace
 // when there is none.
 PyObject *g_workspaces = nullptr, *g_prepare = nullptr;
 
-struct Workspace {
-    void *p;
-    size_t n;
-};
-Workspace workspace(const Tensor &t, lfm2q_stream_t st) {
+Tensor workspace(const Tensor &t) {  // (held by the caller while it is in use)
+    const lfm2q_stream_t st = stream(t);
     require(g_workspaces != nullptr, "lfm2q: the workspace table is not set");
     PyObject *key = Py_BuildValue("(iK)", (int)t.device().index(), (unsigned long long)(uintptr_t)st);
     if (!key) throw std::invalid_argument("");
     PyObject *w = PyDict_GetItemWithError(g_workspaces, key);
     Py_DECREF(key);
     if (!w && PyErr_Occurred()) throw std::invalid_argument("");
-    if (w) {
-        const Tensor &ws = tensor(w, "workspace");
-        return {ws.data_ptr(), (size_t)ws.numel()};
-    }
+    if (w) return tensor(w, "workspace");
     PyObject *dev = PyUnicode_FromFormat("cuda:%d", (int)t.device().index());
     PyObject *made = dev ? PyObject_CallOneArg(g_prepare, dev) : nullptr;
     Py_XDECREF(dev);
     if (!made) throw std::invalid_argument("");
-    const Tensor &ws = tensor(made, "workspace");
-    const Workspace r{ws.data_ptr(), (size_t)ws.numel()};  // the table keeps it alive
+    const Tensor ws = tensor(made, "workspace");
     Py_DECREF(made);
-    return r;
+    return ws;
 }
 
 typedef PyObject *const *Args;
@@ -141,12 +148,11 @@ void gemv(Args a) {
     }
     same_device(W, &x, &y, scale);
     const long rows = integer(a[4]);
-    const auto st = stream(x);
     const float *s = ptr<float>(scale);
     if (int8)
-        run([&] { return lfm2q_gemv_w8(ptr<int8_t>(W), s, ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N, K, rows, st); });
+        run(x, lfm2q_gemv_w8, ptr<int8_t>(W), s, ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N, K, rows);
     else
-        run([&] { return lfm2q_gemv_bf16(ptr<lfm2q_bf16>(W), s, ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N, K, rows, st); });
+        run(x, lfm2q_gemv_bf16, ptr<lfm2q_bf16>(W), s, ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N, K, rows);
 }
 
 // the group size of scales S [R, K / group], and the output width of x [B, K], y [B, N] under epilogue epi
@@ -162,11 +168,8 @@ void w4_run(int fmt, const Tensor &W, const Tensor &S, const Tensor *Z, const Te
     const int64_t N = epi == 1 ? R / 2 : R, B = K ? x.numel() / K : 0;
     require((epi != 1 || R % 2 == 0) && B >= 1 && x.numel() == B * K && y.numel() == B * N, "x [B, K], y [B, N]");
     same_device(W, &S, Z, &x, &y);
-    const auto st = stream(x);
-    run([&] {
-        return lfm2q_gemv_w4(fmt, W.data_ptr(), S.data_ptr(), ptr<int32_t>(Z), ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N,
-                             K, group, epi, st);
-    });
+    run(x, lfm2q_gemv_w4, fmt, W.data_ptr(), S.data_ptr(), ptr<int32_t>(Z), ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N, K,
+        group, epi);
 }
 // (Wp, S, x, y, epi)
 void gemv_w4(Args a) {
@@ -198,8 +201,7 @@ void silu_mul(Args a) {
     const int64_t B = g.numel() / I2;
     require(I2 % 2 == 0 && y.numel() == B * (I2 / 2), "g [B, 2I], y [B, I]");
     same_device(g, &y);
-    const auto st = stream(g);
-    run([&] { return lfm2q_silu_mul(ptr<lfm2q_bf16>(g), ptr<lfm2q_bf16>(y), B, I2 / 2, st); });
+    run(g, lfm2q_silu_mul, ptr<lfm2q_bf16>(g), ptr<lfm2q_bf16>(y), B, I2 / 2);
 }
 
 // ------------------------------------------------------------------------------------------------ GEMMs
@@ -224,18 +226,15 @@ void gemm_i8(Args a) {
     const Tensor &w = tensor(a[2], "w"), &sw = tensor(a[3], "sw"), *b = optional(a[4], "bias"), &y = tensor(a[5], "y");
     same_device(xq, &sx, &w, &sw, b, &y);
     const int gelu = truth(a[6]);
-    const auto st = stream(xq);
+    const int8_t *pq = ptr<int8_t>(xq), *pw = ptr<int8_t>(w);
+    const float *ps = ptr<float>(sx), *psw = ptr<float>(sw);
+    const lfm2q_bf16 *pb = ptr<lfm2q_bf16>(b);
+    lfm2q_bf16 *py = ptr<lfm2q_bf16>(y);
     if (grouped) {
-        run([&] {
-            return lfm2q_gemm_i8_grouped(ptr<int8_t>(xq), ptr<float>(sx), ptr<int8_t>(w), ptr<float>(sw), ptr<lfm2q_bf16>(b),
-                                         ptr<lfm2q_bf16>(y), M, N, K, gelu, st);
-        });
+        run(xq, lfm2q_gemm_i8_grouped, pq, ps, pw, psw, pb, py, M, N, K, gelu);
     } else {  // per token: with the stream's workspace (the K split for shapes with fewer tiles than CUs)
-        const Workspace ws = workspace(xq, st);
-        run([&] {
-            return lfm2q_gemm_i8_ex(ptr<int8_t>(xq), ptr<float>(sx), ptr<int8_t>(w), ptr<float>(sw), ptr<lfm2q_bf16>(b),
-                                    ptr<lfm2q_bf16>(y), M, N, K, gelu, ws.p, ws.n, st);
-        });
+        const Tensor ws = workspace(xq);
+        run(xq, lfm2q_gemm_i8_ex, pq, ps, pw, psw, pb, py, M, N, K, gelu, ws.data_ptr(), (size_t)ws.numel());
     }
 }
 // (xq, sxT, w, sw, bias, yq, ysT, gelu)
@@ -254,11 +253,8 @@ void gemm_i8_q(Args a) {
     if (b) require(b->numel() == N, "bias shape");
     same_device(xq, &sxT, &w, &sw, b, &yq, &ysT);
     const int gelu = truth(a[7]);
-    const auto st = stream(xq);
-    run([&] {
-        return lfm2q_gemm_i8_q(ptr<int8_t>(xq), ptr<float>(sxT), ptr<int8_t>(w), ptr<float>(sw), ptr<lfm2q_bf16>(b),
-                               ptr<int8_t>(yq), ptr<float>(ysT), M, N, K, gelu, st);
-    });
+    run(xq, lfm2q_gemm_i8_q, ptr<int8_t>(xq), ptr<float>(sxT), ptr<int8_t>(w), ptr<float>(sw), ptr<lfm2q_bf16>(b),
+        ptr<int8_t>(yq), ptr<float>(ysT), M, N, K, gelu);
 }
 // (x, w, sw, bias, y, gelu)
 void gemm_w8(Args a) {
@@ -268,12 +264,12 @@ void gemm_w8(Args a) {
     const Tensor &w = tensor(a[1], "w"), &sw = tensor(a[2], "sw"), *b = optional(a[3], "bias"), &y = tensor(a[4], "y");
     same_device(x, &w, &sw, b, &y);
     const int gelu = truth(a[5]);
-    const auto st = stream(x);
-    const Workspace ws = workspace(x, st);  // the K split across workgroups for shapes with few tiles
-    run([&] {
-        return lfm2q_gemm_w8_ex(ptr<lfm2q_bf16>(x), ptr<int8_t>(w), ptr<float>(sw), ptr<lfm2q_bf16>(b), ptr<lfm2q_bf16>(y),
-                                M, N, K, gelu, ws.p, ws.n, st);
-    });
+    const lfm2q_bf16 *px = ptr<lfm2q_bf16>(x), *pb = ptr<lfm2q_bf16>(b);
+    const int8_t *pw = ptr<int8_t>(w);
+    const float *psw = ptr<float>(sw);
+    lfm2q_bf16 *py = ptr<lfm2q_bf16>(y);
+    const Tensor ws = workspace(x);  // the K split across workgroups for shapes with few tiles
+    run(x, lfm2q_gemm_w8_ex, px, pw, psw, pb, py, M, N, K, gelu, ws.data_ptr(), (size_t)ws.numel());
 }
 
 // ------------------------------------------------------------------------------------------------ producers
@@ -282,18 +278,17 @@ void quant_rows(Args a) {
     const Tensor &x = bf16(a[0], "x"), &q = typed(a[1], at::kChar, "q"), &s = typed(a[2], at::kFloat, "s");
     require(x.dim() >= 1, "K must be a multiple of 8");
     const int64_t K = x.size(-1), rows = K ? x.numel() / K : 0;
-    const auto st = stream(x);
     if (s.dim() == 2) {
         require(K % 64 == 0 && K > 0 && s.size(0) == K / 64 && s.size(1) == rows && q.numel() == x.numel(),
                 "grouped shapes");
         same_device(x, &q, &s);
-        run([&] { return lfm2q_quant_groups(ptr<lfm2q_bf16>(x), ptr<int8_t>(q), ptr<float>(s), rows, K, st); });
+        run(x, lfm2q_quant_groups, ptr<lfm2q_bf16>(x), ptr<int8_t>(q), ptr<float>(s), rows, K);
         return;
     }
     require(K % 8 == 0 && K != 0, "K must be a multiple of 8");
     require(q.numel() == x.numel() && s.numel() == rows, "q / s shape");
     same_device(x, &q, &s);
-    run([&] { return lfm2q_quant_rows(ptr<lfm2q_bf16>(x), ptr<int8_t>(q), ptr<float>(s), rows, K, st); });
+    run(x, lfm2q_quant_rows, ptr<lfm2q_bf16>(x), ptr<int8_t>(q), ptr<float>(s), rows, K);
 }
 // per row (1-D s) or per row and 64 columns (2-D s [L / 64, rows])
 int check_qs(const Tensor &q, const Tensor &s, int64_t rows, int64_t L) {
@@ -314,11 +309,8 @@ void add_layernorm_q(Args a) {
     if (x) require(x->numel() == h.numel(), "x shape");
     same_device(h, y, &w, &b, &q, &s, x);
     const float eps = real(a[6]);
-    const auto st = stream(h);
-    run([&] {
-        return lfm2q_add_layernorm_q(ptr<lfm2q_bf16>(h), ptr<lfm2q_bf16>(y), ptr<lfm2q_bf16>(w), ptr<lfm2q_bf16>(b),
-                                     ptr<int8_t>(q), ptr<float>(s), ptr<lfm2q_bf16>(x), rows, D, eps, grouped, st);
-    });
+    run(h, lfm2q_add_layernorm_q, ptr<lfm2q_bf16>(h), ptr<lfm2q_bf16>(y), ptr<lfm2q_bf16>(w), ptr<lfm2q_bf16>(b),
+        ptr<int8_t>(q), ptr<float>(s), ptr<lfm2q_bf16>(x), rows, D, eps, grouped);
 }
 // (h, y, w, q, s, eps, x)
 void add_rmsnorm_q(Args a) {
@@ -332,11 +324,8 @@ void add_rmsnorm_q(Args a) {
     if (x) require(x->numel() == h.numel(), "x shape");
     same_device(h, y, &w, &q, &s, x);
     const float eps = real(a[5]);
-    const auto st = stream(h);
-    run([&] {
-        return lfm2q_add_rmsnorm_q(ptr<lfm2q_bf16>(h), ptr<lfm2q_bf16>(y), ptr<lfm2q_bf16>(w), ptr<int8_t>(q), ptr<float>(s),
-                                   ptr<lfm2q_bf16>(x), rows, H, eps, grouped, st);
-    });
+    run(h, lfm2q_add_rmsnorm_q, ptr<lfm2q_bf16>(h), ptr<lfm2q_bf16>(y), ptr<lfm2q_bf16>(w), ptr<int8_t>(q), ptr<float>(s),
+        ptr<lfm2q_bf16>(x), rows, H, eps, grouped);
 }
 // (g, q, s, x)
 void silu_mul_q(Args a) {
@@ -348,10 +337,7 @@ void silu_mul_q(Args a) {
     const Tensor *x = opt_bf16(a[3], "x");
     if (x) require(x->numel() == rows * I, "x shape");
     same_device(g, &q, &s, x);
-    const auto st = stream(g);
-    run([&] {
-        return lfm2q_silu_mul_q(ptr<lfm2q_bf16>(g), ptr<int8_t>(q), ptr<float>(s), ptr<lfm2q_bf16>(x), rows, I, grouped, st);
-    });
+    run(g, lfm2q_silu_mul_q, ptr<lfm2q_bf16>(g), ptr<int8_t>(q), ptr<float>(s), ptr<lfm2q_bf16>(x), rows, I, grouped);
 }
 
 // ------------------------------------------------------------------------------------------------ module
@@ -375,6 +361,9 @@ PyObject *entry(PyObject *, Args args, Py_ssize_t n) {
         F(args);
     } catch (const std::invalid_argument &) {  // the Python error is already set
         if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "invalid argument");
+        return nullptr;
+    } catch (const c10::Error &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
         return nullptr;
     } catch (const std::exception &e) {
         PyErr_SetString(PyExc_RuntimeError, e.what());
