@@ -209,8 +209,9 @@ __device__ __forceinline__ float silu_f32(float g) {
 // bf16(silu) of 8 bf16 values (one 16-byte vector), as fp32: silu_f32's bits after the rounding at a third of its
 // instructions. For |g| < 32 neither the clamp, the scaling nor the compensation of the exponent's argument matters to the
 // rounded result (equal to silu_f32's for every bf16 of that range); a vector with a larger value or a NaN takes silu_f32.
-// silu_mul_q, bound by its vector operations, with this and max8 in place of LDS permutes, 8192 wide on MI355X: 4096 rows
-// 47.6 -> 37.8 us, 2048 27.9 -> 21.6, 461 10.8 -> 8.7.
+// The larger values' side is a branch (left to itself the compiler computed both sides and selected, which took 4096 x 2048
+// 12.5 -> 14.9 us; 10.7 so). silu_mul_q, bound by its vector operations, with this and max8 in place of LDS permutes, 8192
+// wide on MI355X: 4096 rows 43.6 -> 37.0 us, 2048 25.9 -> 20.0, 461 8.9 -> 7.5.
 typedef unsigned short v2us __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void silu8_bf16(v4i gv, float (&o)[8]) {
 #pragma clang fp contract(off)
@@ -223,6 +224,7 @@ __device__ __forceinline__ void silu8_bf16(v4i gv, float (&o)[8]) {
         m = __builtin_elementwise_max(m, __builtin_bit_cast(v2us, gv[j] & 0x7fff7fff));
     }
     if (__builtin_expect(max((int)m[0], (int)m[1]) >= 0x4200, 0)) {  // |g| >= 32, inf or NaN
+        asm volatile("");  // not to be computed beside the other side
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] = rbf(silu_f32(g[e]));
     } else {

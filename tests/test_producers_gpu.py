@@ -213,6 +213,22 @@ def test_silu_mul_q_workgroup_form_matches_wavefront_form(E, tune, rows, I, grou
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))  # bit patterns
 
 
+@pytest.mark.parametrize("rows,I", [(5, 8192), (9, 2048), (70, 1152), (3, 64)])
+def test_silu_mul_q_large_gates_beside_small_ones(E, D, rows, I):
+    """Gates past the short form of SiLU (|g| >= 32, infinite too) in some lanes of a wavefront: bf16 x is silu_mul's."""
+    bits = rand_bf16(rows * I, (rows, 2 * I), 2.0)
+    big = np.random.default_rng(I).random(bits.shape) < 0.02
+    bits[big] = (bits[big] & 0x8000) | 0x4280  # +-64
+    bits[0, 3] = 0x7F80  # inf (its product with a bf16 value is inf; quantized values are not compared)
+    g = dev_bf16(bits)
+    a = torch.empty(rows, I, device="cuda", dtype=torch.bfloat16)
+    D.silu_mul(g, a)
+    for grouped in (False, True):
+        x = torch.empty_like(a)
+        E.silu_mul_q(g, *qs_buffers(rows, I, grouped), x=x)
+        assert torch.equal(x.view(torch.int16), a.view(torch.int16))
+
+
 def test_silu_mul_q_non_grouped_length(E, D):
     """A length that is not a multiple of 64 (4304, the vision MLP width) is accepted per row, and rejected grouped."""
     rows, I = 6, 4304
