@@ -86,8 +86,8 @@ class DecodeOps:
         if not (S.dim() == 2 and S.size(0) == R and S.size(1) >= 1 and K % S.size(1) == 0):
             raise RuntimeError("S must be [N, K / group]")
         group = K // S.size(1)
-        if group % 32:
-            raise RuntimeError("group size must be a multiple of 32")
+        if group <= 0 or group % 32:
+            raise RuntimeError("group size must be a positive multiple of 32")
         return group
 
     def silu_mul(self, g, y):

@@ -52,3 +52,26 @@ def test_a_tensor_without_a_pointer_is_an_error(op):
 
     with pytest.raises(RuntimeError, match="data pointer"):
         torch.func.vmap(call)(Claim(3, *shape, dt=dt))
+
+
+@pytest.mark.parametrize("op", ["gemv_w4", "gemv_w4z"])
+def test_w4_weights_without_columns_are_an_error(op):
+    """K = 0 makes a group of no weights: refused before anything is divided by it."""
+    from lfm2opt import _capi
+
+    x, y = C(1, 0), C(1, 8)
+    args = {"gemv_w4": (C(8, 0, dt=torch.uint8), C(8, 1, dt=F32), x, y, 0),
+            "gemv_w4z": (C(8, 0, dt=torch.int32), C(8, 1, dt=torch.float16), C(8, 1, dt=torch.int32), x, y, 0)}[op]
+    with pytest.raises(RuntimeError, match="positive multiple of 32"):
+        getattr(_capi.native(), op)(*args)
+
+
+@pytest.mark.parametrize("op", ["gemv_w4_rmsnorm", "gemv_conv_rmsnorm"])
+def test_w4z_weights_without_columns_are_an_error_with_a_norm(op):
+    from lfm2opt.kernels import ext
+
+    W, S, Z = C(24, 0, dt=torch.int32), C(24, 1, dt=torch.float16), C(24, 1, dt=torch.int32)
+    args = {"gemv_w4_rmsnorm": (W, S, Z, C(1, 0), C(0), 1e-5, C(1, 24)),
+            "gemv_conv_rmsnorm": (W, S, Z, C(1, 0), C(0), 1e-5, C(3, 1, 8), C(3, 8), None, C(2, dt=torch.int64), C(1, 8))}[op]
+    with pytest.raises(RuntimeError, match="positive multiple of 32"):
+        getattr(ext(), op)(*args)
