@@ -159,7 +159,7 @@ void gemv(Args a) {
 int64_t w4_group(const Tensor &S, int64_t R, int64_t K) {
     require(S.dim() == 2 && S.size(0) == R && S.size(1) >= 1 && K % S.size(1) == 0, "S must be [N, K / group]");
     const int64_t group = K / S.size(1);
-    require(group > 0 && group % 32 == 0, "group size must be a positive multiple of 32");  // (0: a weight without columns)
+    require(group > 0 && group % 32 == 0, "group size must be a multiple of 32");  // (0: a weight without columns)
     return group;
 }
 void w4_run(int fmt, const Tensor &W, const Tensor &S, const Tensor *Z, const Tensor &x, const Tensor &y, int64_t R,

@@ -87,7 +87,7 @@ class DecodeOps:
             raise RuntimeError("S must be [N, K / group]")
         group = K // S.size(1)
         if group <= 0 or group % 32:
-            raise RuntimeError("group size must be a positive multiple of 32")
+            raise RuntimeError("group size must be a multiple of 32")
         return group
 
     def silu_mul(self, g, y):

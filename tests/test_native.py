@@ -62,7 +62,7 @@ def test_w4_weights_without_columns_are_an_error(op):
     x, y = C(1, 0), C(1, 8)
     args = {"gemv_w4": (C(8, 0, dt=torch.uint8), C(8, 1, dt=F32), x, y, 0),
             "gemv_w4z": (C(8, 0, dt=torch.int32), C(8, 1, dt=torch.float16), C(8, 1, dt=torch.int32), x, y, 0)}[op]
-    with pytest.raises(RuntimeError, match="positive multiple of 32"):
+    with pytest.raises(RuntimeError, match="group size must be a multiple of 32"):
         getattr(_capi.native(), op)(*args)
 
 
@@ -73,5 +73,5 @@ def test_w4z_weights_without_columns_are_an_error_with_a_norm(op):
     W, S, Z = C(24, 0, dt=torch.int32), C(24, 1, dt=torch.float16), C(24, 1, dt=torch.int32)
     args = {"gemv_w4_rmsnorm": (W, S, Z, C(1, 0), C(0), 1e-5, C(1, 24)),
             "gemv_conv_rmsnorm": (W, S, Z, C(1, 0), C(0), 1e-5, C(3, 1, 8), C(3, 8), None, C(2, dt=torch.int64), C(1, 8))}[op]
-    with pytest.raises(RuntimeError, match="positive multiple of 32"):
+    with pytest.raises(RuntimeError, match="group size must be a multiple of 32"):
         getattr(ext(), op)(*args)
