@@ -155,6 +155,12 @@ void gemv(Args a) {
         run(x, lfm2q_gemv_bf16, ptr<lfm2q_bf16>(W), s, ptr<lfm2q_bf16>(x), ptr<lfm2q_bf16>(y), B, N, K, rows);
 }
 
+// the epilogue of an INT4 GEMV: 0, 1 or 2, as any number
+long epilogue(PyObject *o) {
+    if (!PyFloat_Check(o)) return integer(o);
+    const double v = PyFloat_AS_DOUBLE(o);
+    return v == 0.0 || v == 1.0 || v == 2.0 ? (long)v : -1;
+}
 // the group size of scales S [R, K / group], and the output width of x [B, K], y [B, N] under epilogue epi
 int64_t w4_group(const Tensor &S, int64_t R, int64_t K) {
     require(S.dim() == 2 && S.size(0) == R && S.size(1) >= 1 && K % S.size(1) == 0, "S must be [N, K / group]");
@@ -178,7 +184,7 @@ void gemv_w4(Args a) {
             "Wp: contiguous uint8 [N, K/2]");
     require(S.is_cuda() && S.is_contiguous() && S.scalar_type() == at::kFloat, "S: contiguous fp32 [N, K/128]");
     const int64_t R = W.size(0), K = W.size(1) * 2;
-    w4_run(0, W, S, nullptr, x, y, R, K, w4_group(S, R, K), integer(a[4]));
+    w4_run(0, W, S, nullptr, x, y, R, K, w4_group(S, R, K), epilogue(a[4]));
 }
 // (qweight, scales, qzeros, x, y, epi)
 void gemv_w4z(Args a) {
@@ -191,7 +197,7 @@ void gemv_w4z(Args a) {
     require(Z.is_cuda() && Z.is_contiguous() && Z.scalar_type() == at::kInt && Z.dim() == 2 && Z.size(0) == R &&
                 Z.size(1) == (G + 7) / 8,
             "qzeros: contiguous int32 [N, ceil(K/group/8)]");
-    w4_run(1, W, S, &Z, x, y, R, K, group, integer(a[5]));
+    w4_run(1, W, S, &Z, x, y, R, K, group, epilogue(a[5]));
 }
 // (g, y)
 void silu_mul(Args a) {

@@ -75,3 +75,21 @@ def test_w4z_weights_without_columns_are_an_error_with_a_norm(op):
             "gemv_conv_rmsnorm": (W, S, Z, C(1, 0), C(0), 1e-5, C(3, 1, 8), C(3, 8), None, C(2, dt=torch.int64), C(1, 8))}[op]
     with pytest.raises(RuntimeError, match="group size must be a multiple of 32"):
         getattr(ext(), op)(*args)
+
+
+@pytest.mark.parametrize("op", ["gemv_w4", "gemv_w4z"])
+def test_w4_epilogue_as_a_float(op):
+    """epi = 1.0 is 1 (the call goes on to read the pointers); another number is refused as an epilogue."""
+    from lfm2opt import _capi
+
+    shape, dt, args = CALLS[op]
+
+    def call(x, epi):
+        a = args(x)
+        getattr(_capi.native(), op)(*a[:-2], C(1, 4), epi)
+        return x
+
+    with pytest.raises(RuntimeError, match="data pointer"):
+        torch.func.vmap(lambda x: call(x, 1.0))(Claim(3, *shape, dt=dt))
+    with pytest.raises(RuntimeError, match="epi 0"):
+        call(C(*shape), 1.5)
