@@ -238,3 +238,15 @@ def test_generate_stop_at_eos():
     # EOS as the very first token: no replay at all
     dec.eos = torch.tensor([free[0]])
     assert dec.generate(ids, 12, stop_at_eos=True, graph=False).shape == (1, 6)
+
+
+def test_a_decoder_without_layers():
+    """The embedding, its norm and the head alone: a state without caches clears."""
+    net = tiny_lfm2(seed=15, layer_types=("conv",))
+    lin = TorchLinears(decode_weights(net))
+    net.config.num_hidden_layers = 0
+    dec = StaticDecoder(net, bucket=8, keep_logits=True, linears=lin)
+    ids = torch.randint(3, net.config.vocab_size, (2, 3), generator=torch.Generator().manual_seed(3))
+    h = net.model.embed_tokens.weight[ids]
+    want = torch.nn.functional.linear(net.model.embedding_norm(h), net.lm_head.weight)
+    assert rel_err(step_logits(dec, ids), want.detach()) < 1e-5
