@@ -250,3 +250,15 @@ def test_a_decoder_without_layers():
     h = net.model.embed_tokens.weight[ids]
     want = torch.nn.functional.linear(net.model.embedding_norm(h), net.lm_head.weight)
     assert rel_err(step_logits(dec, ids), want.detach()) < 1e-5
+
+
+def test_conv_taps_are_on_16_bytes_wherever_the_weight_is():
+    """The convolution kernels read the taps in 8- and 16-byte vectors; with one tap the transposed weight is the weight
+    itself, which may lie anywhere."""
+    net = tiny_lfm2(seed=17, layer_types=("conv",))
+    conv, H = net.model.layers[0].conv.conv, net.config.hidden_size
+    buf = torch.randn(H + 1)
+    conv.weight = torch.nn.Parameter(buf[1:].view(H, 1, 1), requires_grad=False)
+    net.config.conv_L_cache = 1
+    dec = StaticDecoder(net, bucket=8, linears=TorchLinears(decode_weights(net)))
+    assert dec.conv_wt[0].data_ptr() % 16 == 0 and torch.equal(dec.conv_wt[0][0], buf[1:])
