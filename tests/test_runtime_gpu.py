@@ -14,7 +14,7 @@ import copy
 import pytest
 import torch
 
-from lfm2_tiny import reference_logits, step_logits, tiny_lfm2
+from lfm2_tiny import TorchLinears, reference_logits, step_logits, tiny_lfm2
 
 pytestmark = pytest.mark.gpu
 
@@ -88,6 +88,38 @@ def test_decode_step_against_transformers(nets, mode, B, paths):
     err = rel_err(got, want)
     print(f"runtime {mode} B={B}: max |err| / max |ref| = {err:.2e}")
     assert err <= TOL
+
+
+class ViewLinears(TorchLinears):
+    """Linears whose results are views one column into a wider matrix (not contiguous, at batch 1 contiguous but off 16
+    bytes), and logits in fp32."""
+
+    def norm_fusable(self, B, key):
+        return False
+
+    def linear(self, x, key, bias=None):
+        if key[0] == "head":
+            return x.float() @ self.w[key].float().t()
+        y = super().linear(x, key, bias)
+        wide = y.new_full((y.shape[0], y.shape[1] + 3), float("nan"))
+        wide[:, 1:-2] = y
+        return wide[:, 1:-2]
+
+
+@pytest.mark.parametrize("B", [1, 2])
+def test_linears_that_return_views_and_fp32_logits(nets, B):
+    """A decoder on linears of the caller's: their results need not have the layout or the logits the type that the
+    step's kernels read. TOL against transformers on the same BF16 weights."""
+    from lfm2opt.runtime import StaticDecoder, decode_weights
+
+    _, gnet = nets
+    dec = StaticDecoder(gnet, bucket=32, keep_logits=True, linears=ViewLinears(decode_weights(gnet)))
+    ids = torch.randint(3, gnet.config.vocab_size, (B, 9), generator=torch.Generator().manual_seed(5))
+    print(f"linears that return views, B={B}", flush=True)
+    got = step_logits(dec, ids)
+    assert rel_err(got, reference_logits(copy.deepcopy(gnet).to("cpu", torch.float32), ids)) <= TOL
+    out = dec.generate(ids, 3, graph=False)
+    assert torch.equal(out[:, 9].cpu(), got[:, -1].index_fill(-1, dec.eos.cpu(), float("-inf")).argmax(-1))
 
 
 def test_generate_graph_equals_eager(nets):
