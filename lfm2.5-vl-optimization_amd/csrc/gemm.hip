@@ -724,8 +724,7 @@ __global__ __launch_bounds__(GT * KSP) __attribute__((amdgpu_waves_per_eu(gemm_w
 // barriers; each fold runs beside the next group's MFMAs (two int32 buffers), half of it after each; the next stage's
 // barrier and fragment reads come before a stage's arithmetic (two register sets). What is left bounds it: the weights' and
 // scales' latency from HBM (the loads alone take two thirds of the time) and ~32 vector operations a group. MI355X, us, 461
-// tokens x K x N: 8192 x 2048 31.5 -> 26.5, 2048 x 2048 10.2 -> 9.4, 2048 x 3072 (128 x 64 tiles before) 14.3 -> 11.8,
-// 2048 x 6144 (128 x 128) 20.8 -> 18.6. Deeper rings with one workgroup a CU (4 groups a stage, 6 or 8 slots), 8 wavefronts
+// tokens x K x N: 8192 x 2048 29.5 -> 26.7, 2048 x 2048 10.1 -> 9.4, 2048 x 3072 (128 x 64 tiles before) 14.2 -> 12.0. Deeper rings with one workgroup a CU (4 groups a stage, 6 or 8 slots), 8 wavefronts
 // of 32 x 16 blocks and 128-byte rows were no faster.
 template <int OUT>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_i8_few_kernel(
@@ -1887,14 +1886,20 @@ void launch_gemm_grouped(const int8_t *A, const int8_t *B, const float *sxT, con
                                                                                    YsT);
         return;
     }
-    // bf16 output with K >= 2048 and at most three 64 x 64 tiles a CU: the kernel for few tiles, whatever tile the model
-    // above picks (it was fitted without it). Measured on MI355X over 18 such shapes 2 to 25 % faster (600 x 8192 x 2048 44.1
-    // -> 33.1 us, 1500 x 2048 x 2048 18.8 -> 18.4) but for 100 x 2048 x 16384 (15.2 -> 15.5); past three tiles a CU (600 x
-    // 2048 x 6144 21.0 -> 21.9) and for short K (1024 x 1152 x 1152 7.75 -> 8.2) it loses. LFM2Q_GEMM_GSEQ = 2 forces it.
+    // bf16 output, K >= 2048: the kernel for few tiles up to two 64 x 64 tiles a CU, whatever tile the model above picks (it
+    // was fitted without it), and up to three where that is 128 x 128, one a CU. Measured on MI355X against the model's
+    // tile over 190 shapes: 5 to 24 % faster there (tokens x K x N: 20 x 2048 x 2048 9.7 -> 8.9 us, 600 x 8192 x 2048 43.9 ->
+    // 33.5, 1500 x 8192 x 2048 64.7 -> 59.0); where the model takes 64 x 64 tiles at more than two a CU they are 1 to 14 %
+    // faster than it (800 x 2048 x 3072 16.9 against 18.1, 333 x 2048 x 6144 16.0 against 17.8), past three 128 x 128 tiles
+    // are (2 to 9 %). Over wide weights a second row of tiles soon costs more than it saves: 2048 x 16384 at 65 rows 14.4 ->
+    // 12.4, 100 14.8 -> 14.2, 128 15.0 -> 15.6; 2048 x 14336 at 128 14.5 -> 13.1 or 15.6, by where the weights lie; 4096 x
+    // 16384 at 72 25.5 -> 26.0, 128 26.4 -> 32.3. Short K loses past one tile a CU (1024 x 1152 x 1152 7.75 -> 8.2). LFM2Q_GEMM_GSEQ = 2 forces it.
     if constexpr (!out_q8(OUT)) {
-        const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64);
+        const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64), cus = device_cus();
         const bool forced = three || (knob_int(KNOB_GEMM_BM, 0) && knob_int(KNOB_GEMM_BN, 0));
-        if (gseq >= 0 ? gseq == 2 : !forced && K >= 2048 && t64 <= 3L * device_cus()) {
+        const bool few = K >= 2048 && t64 <= (t.bm == 128 && t.bn == 128 ? 3 : 2) * cus &&
+                         (N < 14336 || M <= (K > 2048 ? 64 : 96));
+        if (gseq >= 0 ? gseq == 2 : !forced && few) {
             gemm_i8_few_kernel<OUT><<<dim3(t64), GT, 0, st>>>(A, B, sxT, sw, bias, Y, M, N, K, sh);
             return;
         }
