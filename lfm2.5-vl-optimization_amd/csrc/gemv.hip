@@ -41,12 +41,16 @@ namespace {
 // i.e. vectors XL (l + 64 u) + q. NORM: x is the RMSNorm of the row h with weight nw, computed here exactly as
 // add_rmsnorm_q computes it (rmsnorm.hpp), so the GEMV of the normalized row equals add_rmsnorm_q followed by the
 // GEMV bit for bit: the sum of squares is taken in add_rmsnorm_q's order -- lane l sums vectors c 64 + l, c < CH =
-// CPL XL -- by loading those vectors as well (they are in the L1 with the lane's own; fetching them from the lanes that
-// hold them took 8 LDS permutes a vector; for XL = 1 the two layouts coincide), then x = bf16(w bf16(h rs))
+// CPL XL. For XL = 1 that is the lane's own layout. For XL = 2 with 2 or 4 chunks those vectors are loaded as well (they are in
+// the L1 with the lane's own; 6144 x 2048 INT8 5.5 -> 4.9 us, 2048 x 4096 6.3 -> 5.6 against the permutes); with 1 or 8 they
+// are fetched from the lanes that hold them by 8 LDS permutes a vector (vector c 64 + l is register [c / 2][l % 2] of lane 32
+// (c % 2) + l / 2), where the loads were slower (65536 x 1024 12.3 -> 13.0, 6144 x 1024 3.8 -> 4.0, SwiGLU 8192 x 8192 32.6 ->
+// 33.9). Then x = bf16(w bf16(h rs))
 // elementwise in the kernel's own layout. Needs K = 64 PER CPL exactly (every vector in range).
 template <int PER, int XL, int CPL, bool NORM>
 struct XLoadB1 {
-    v4i hv[CPL][XL], wv[CPL][XL], sv[XL == 1 ? 1 : CPL * XL];
+    static constexpr bool OWN = XL == 1, LOADS = !OWN && (CPL == 2 || CPL == 4);  // where the sum's vectors come from
+    v4i hv[CPL][XL], wv[CPL][XL], sv[LOADS ? CPL * XL : 1];
     // NORM: the row and the norm weight, in flight before the caller issues its weight loads
     __device__ __forceinline__ void issue(const uint16_t *__restrict__ x, const uint16_t *__restrict__ nw, int lane) {
         if constexpr (NORM) {
@@ -57,7 +61,7 @@ struct XLoadB1 {
                     hv[u][q] = ld16(x + (size_t)(lane + 64 * u) * PER + 8 * q);
                     wv[u][q] = ld16(nw + (size_t)(lane + 64 * u) * PER + 8 * q);
                 }
-            if constexpr (XL > 1)
+            if constexpr (LOADS)
 #pragma unroll
                 for (int c = 0; c < CPL * XL; ++c) sv[c] = ld16(x + (size_t)(c * 64 + lane) * 8);
         }
@@ -72,7 +76,22 @@ struct XLoadB1 {
         } else {
             float ss = 0.f;
 #pragma unroll
-            for (int c = 0; c < CPL * XL; ++c) ss = sumsq8(XL == 1 ? hv[c][0] : sv[c], ss);
+            for (int c = 0; c < CPL * XL; ++c) {
+                if constexpr (OWN) {
+                    ss = sumsq8(hv[c][0], ss);
+                } else if constexpr (LOADS) {
+                    ss = sumsq8(sv[c], ss);
+                } else {
+                    const int src = 32 * (c & 1) + (lane >> 1);
+                    v4i g;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int a = __shfl(hv[c >> 1][0][j], src), b = __shfl(hv[c >> 1][1][j], src);
+                        g[j] = (lane & 1) ? b : a;
+                    }
+                    ss = sumsq8(g, ss);
+                }
+            }
             const float rs = rms_scale(wave_sum(ss), K, eps);
 #pragma unroll
             for (int u = 0; u < CPL; ++u)
