@@ -6,7 +6,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# attn_step: the output is one bf16 rounding (2^-9 of the value) of fp32 sums over at most 4,096 positions of values up
+# attn_step: the output is one bf16 rounding (2^-9 of the value) of fp32 sums over at most 16,384 positions (2^-10 in the worst order) of values up
 # to max |v|; q stays fp32, so its own error is the exp2 of an fp32 score (|score| < 2^6: 2^-18). 2^-8 of the largest
 # value covers all of it.
 ATTN_TOL = 2.0 ** -8
@@ -32,7 +32,11 @@ def attention_reference(qkv, qk_w, rope, pos, k, v, scale, eps):
 @pytest.mark.parametrize("G", [1, 2, 4, 8])
 @pytest.mark.parametrize("B,max_len,positions", [(1, 8, (0, 3, 7)), (2, 256, (0, 31, 255)), (1, 264, (256, 263)),
                                                  (3, 512, (255, 256, 511)), (1, 1032, (767, 768, 1031)),
-                                                 (1, 4096, (2047, 4095)), (40, 1280, (0, 300, 1279))])
+                                                 (1, 4096, (2047, 4095)), (40, 1280, (0, 300, 1279)),
+                                                 # eight heads a workgroup (G = 8); splits of two and four chunks, at and
+                                                 # beside their edges; more than 16 and up to 64 splits to combine
+                                                 (65, 512, (255, 256, 511)), (16, 4096, (511, 512, 1023, 1024, 1500, 4095)),
+                                                 (1, 8192, (4095, 4096, 8191)), (1, 16384, (12288, 16383))])
 def test_attn_step(cuda, G, B, max_len, positions):
     from lfm2opt.kernels import ext
 
