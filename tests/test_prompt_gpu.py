@@ -29,9 +29,13 @@ def reference(qkv, qk_w, rope, nkv, scale, eps):
     return torch.matmul(torch.softmax(s, -1), vr.transpose(1, 2)).transpose(1, 2).reshape(B, T, -1), k, v
 
 
-@pytest.mark.parametrize("G", [1, 2, 4, 8])
-@pytest.mark.parametrize("B,T,max_len", [(1, 1, 8), (2, 31, 40), (1, 33, 256), (3, 64, 64), (1, 65, 72), (2, 129, 256),
-                                         (1, 500, 512)])
+SHAPES = [(1, 1, 8), (2, 31, 40), (1, 33, 256), (3, 64, 64), (1, 65, 72), (2, 129, 256), (1, 500, 512)]
+# with 2 kv heads on 256 CUs: more tiles of positions than a round of the work order holds, so rounds of falling order and
+# a shorter last one (per G: tiles of 128, 64, 32 and 32 positions)
+ROUNDS = [(1, 64, 300, 304), (2, 64, 300, 304), (4, 32, 430, 432), (8, 16, 300, 304)]
+
+
+@pytest.mark.parametrize("G,B,T,max_len", [(G, *s) for G in (1, 2, 4, 8) for s in SHAPES] + ROUNDS)
 def test_prompt_attn(cuda, G, B, T, max_len):
     from lfm2opt.kernels import ext, int8_ext
 
@@ -47,7 +51,7 @@ def test_prompt_attn(cuda, G, B, T, max_len):
     want, kn, vn = reference(qkv, qk_w, rope, nkv, scale, eps)
     k = torch.full((B, nkv, 64, max_len), 7.0, dtype=BF, device=cuda)
     v = torch.full((B, nkv, max_len, 64), 7.0, dtype=BF, device=cuda)
-    out = torch.empty(B * T, nh * 64, dtype=BF, device=cuda)
+    out = torch.full((B * T, nh * 64), float("nan"), dtype=BF, device=cuda)  # a tile left out stays NaN
     args = (qk_w.to(cuda), rope.to(cuda))
     ext().prompt_attn(qkv.to(cuda), *args, k, v, out, scale, eps)
     err = (out.cpu().double().view_as(want) - want).abs()
@@ -58,7 +62,7 @@ def test_prompt_attn(cuda, G, B, T, max_len):
     assert ((kc[..., :T].double() - kn.permute(0, 2, 3, 1)).abs() <= 2.0 ** -7 * kn.abs().max()).all()
     assert (kc[..., T:] == 7).all() and (vc[:, :, T:] == 7).all()
     # the quantized form is quant_groups of the bf16 form
-    q, s = torch.empty(B * T, nh * 64, dtype=torch.int8, device=cuda), torch.empty(nh, B * T, device=cuda)
+    q, s = torch.empty(B * T, nh * 64, dtype=torch.int8, device=cuda), torch.full((nh, B * T), float("nan"), device=cuda)
     ext().prompt_attn(qkv.to(cuda), *args, k, v, (q, s), scale, eps)
     q2, s2 = torch.empty_like(q), torch.empty_like(s)
     int8_ext().quant_rows(out, q2, s2)
