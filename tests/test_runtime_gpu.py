@@ -29,6 +29,12 @@ def nets(cuda):
     return net, copy.deepcopy(net).to(cuda, torch.bfloat16)
 
 
+@pytest.fixture(scope="module")
+def wide_heads(cuda):
+    """Heads of 128, which the attention kernels do not take."""
+    return tiny_lfm2(seed=23, heads=2, kv_heads=1).to(cuda, torch.bfloat16)
+
+
 def path_weight(lin, key, B):
     """The fp32 weight (CPU) that the call for key at batch B multiplies."""
     from lfm2opt.quant import dequantize_int4
@@ -214,27 +220,33 @@ def prefill_oracle(gpu_net, dec, B, w8a8):
                                                           ("cublas", {"fused_prefill": True}, "64", 1024),
                                                           ("int8", {"prefill_int8": True}, "64", 8),
                                                           ("cublas", {"fused_prefill": True}, "64", 8)])
-def test_batched_prefill(nets, mode, flags, group, blocks_from, monkeypatch):
+def test_batched_prefill(nets, wide_heads, mode, flags, group, blocks_from, monkeypatch):
     """The whole prompt in one pass (W8A8 with the fused quantizing producers, or BF16 GEMMs): the last position's
     logits against transformers' forward on the weights the GEMMs read (bar PREFILL_TOL: the W8A8 form also
     quantizes every GEMM input to int8), and the k / v rows and conv states it leaves in the static buffers against
     the ones the per-token prefill leaves (same bar: a row at the wrong position or head is off by ~100 %); then
-    decoding continues from that state. blocks_from 8 takes the prompt attention in four blocks of positions (the
-    form prompts of 1024 positions and more take)."""
+    decoding continues from that state. blocks_from 8 runs the PyTorch forms that other shapes than the kernels' take
+    (heads of 128, and the convolution's and the tail's by switch), the prompt attention in four blocks of positions
+    (as prompts of 1024 positions and more take it)."""
     from lfm2opt.runtime import StaticDecoder
 
-    _, gnet = nets
+    fused = blocks_from > 21
+    gnet = nets[1] if fused else wide_heads
     B, T = 2, 21
     ids = torch.randint(3, gnet.config.vocab_size, (B, T), generator=torch.Generator().manual_seed(11))
     monkeypatch.setenv("LFM2_INT8_GROUP", group)  # W8A8 activation scales per 64-channel group, or per token
     dec = StaticDecoder(gnet, bucket=32, keep_logits=True, gemv=mode, **flags)
     dec.prompt_blocks_from = blocks_from
+    dec.fused_conv, dec.fused_tail = dec.fused_conv and fused, dec.fused_tail and fused
     print(f"batched prefill {mode} {flags} group {group} blocks_from {blocks_from}", flush=True)
     first, s = dec.prefill(ids, 6)
     want = reference_logits(prefill_oracle(gnet, dec, B, "prefill_int8" in flags), ids)[:, -1]
     err = rel_err(dec.last_prefill_logits.cpu(), want)
     step = StaticDecoder(gnet, bucket=32, gemv=mode)
+    step.fused_conv, step.fused_tail = dec.fused_conv, dec.fused_tail
     _, s2 = step.prefill(ids, 6, graph=False)
+    for st in (s, s2):
+        assert (st.attn_ws is not None) == (st.tail_ws is not None) == dec.fused_conv == fused
     errs = {f"k{i}": rel_err(s.k[i][..., :T].float().cpu(), s2.k[i][..., :T].float().cpu()) for i in s.k}
     errs.update({f"v{i}": rel_err(s.v[i][:, :, :T].float().cpu(), s2.v[i][:, :, :T].float().cpu()) for i in s.v})
     errs.update({f"conv{i}": rel_err(s.conv[i].float().cpu(), s2.conv[i].float().cpu()) for i in s.conv})
