@@ -214,17 +214,13 @@ __global__ __launch_bounds__(256) void attn_step_kernel(const uint16_t *__restri
 #pragma unroll 8
         for (int r = 0; r < 32; ++r) o += red[(r * G + g) * HD + d];
         const float lt = (wl[0][g] + wl[1][g]) + (wl[2][g] + wl[3][g]);
-        if (splits == 1) {
+        if (G > 1 || splits == 1) {
             out[((size_t)b * nh + h0 + g) * HD + d] = (uint16_t)f2bf(o / lt);
         } else {
-            // partial (head, split): 64 unnormalized outputs, then its maximum and row sum
-            float *pp = part + (((size_t)b * nh + h0 + g) * splits + split) * (HD + 2);
-            float mg = m[0];
-#pragma unroll
-            for (int k = 1; k < G; ++k)
-                if (k == g) mg = m[k];
+            // partial (head, split): 64 unnormalized outputs, then its maximum and row sum (several splits: G = 1)
+            float *pp = part + (((size_t)b * nh + h0) * splits + split) * (HD + 2);
             pp[d] = o;
-            if (d == 0) pp[HD] = mg, pp[HD + 1] = lt;
+            if (d == 0) pp[HD] = m[0], pp[HD + 1] = lt;
         }
     }
 }
@@ -267,7 +263,8 @@ struct AttnShape {
 // First the query heads of a kv head over workgroups (each reads the kv head's cache again, from the L2) while that
 // leaves no more workgroups than CUs: the arithmetic of four heads is half of a workgroup's time. Then the positions:
 // about two workgroups a CU and at most 64 splits (the combine pass's lanes), but no split for two chunks or where
-// fewer than four would come of it, which the combine pass (a launch, ~2.5 us) outweighs. MI355X, 32 heads over 8, us in
+// fewer than four would come of it, which the combine pass (a launch, ~2.5 us) outweighs. Several heads a workgroup mean more
+// than half as many workgroups as CUs, so at most three splits: they never come with several splits. MI355X, 32 heads over 8, us in
 // a graph (rows, positions: heads per workgroup 1 / 2 / 4): 1, 200 4.9 / 5.6 / 7.0; 1, 400 6.5 / 7.6 / 10.0 (two splits
 // 7.4 / 8.0 / 9.5); 1, 3001 in 16 splits 8.7 / 8.8 / 10.3 (8 splits 9.8, one 23.7); 16, 1000 13.5 / 13.3 / 17.7 (two
 // splits 18.1 / 14.3 / 15.6); 64, 2000 90 / 63 / 58 (two splits 100 / 69 / 62).
@@ -276,7 +273,7 @@ inline AttnShape attn_shape(int B, int nkv, int grp, int max_len) {
     int heads = grp;
     while (heads > 1 && (long)B * nkv * (grp / heads) * 2 <= device_cus()) heads /= 2;
     const int want = (int)std::min<long>(64, 2 * device_cus() / ((long)B * nkv * (grp / heads)));
-    int splits = total <= 2 || want < 4 ? 1 : std::min(total, want);
+    int splits = heads > 1 || total <= 2 || want < 4 ? 1 : std::min(total, want);
     const int chunks = (total + splits - 1) / splits;
     splits = (total + chunks - 1) / chunks;
     return {chunks, splits, heads};

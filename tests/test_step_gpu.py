@@ -6,9 +6,9 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# attn_step: the output is one bf16 rounding (2^-9 of the value) of fp32 sums over at most 16,384 positions (2^-10 in the worst order) of values up
-# to max |v|; q stays fp32, so its own error is the exp2 of an fp32 score (|score| < 2^6: 2^-18). 2^-8 of the largest
-# value covers all of it.
+# attn_step: the output is one bf16 rounding (2^-9 of the value) of fp32 sums over at most 16,384 positions (2^-10 in the
+# worst order) of values up to max |v|; q stays fp32, so its own error is the exp2 of an fp32 score (|score| < 2^6: 2^-18).
+# 2^-8 of the largest value covers all of it.
 ATTN_TOL = 2.0 ** -8
 
 
