@@ -724,8 +724,9 @@ __global__ __launch_bounds__(GT * KSP) __attribute__((amdgpu_waves_per_eu(gemm_w
 // barriers; each fold runs beside the next group's MFMAs (two int32 buffers), half of it after each; the next stage's
 // barrier and fragment reads come before a stage's arithmetic (two register sets). What is left bounds it: the weights' and
 // scales' latency from HBM (the loads alone take two thirds of the time) and ~32 vector operations a group. MI355X, us, 461
-// tokens x K x N: 8192 x 2048 29.5 -> 26.7, 2048 x 2048 10.1 -> 9.4, 2048 x 3072 (128 x 64 tiles before) 14.2 -> 12.0. Deeper rings with one workgroup a CU (4 groups a stage, 6 or 8 slots), 8 wavefronts
-// of 32 x 16 blocks and 128-byte rows were no faster.
+// tokens x K x N: 8192 x 2048 29.5 -> 26.7, 2048 x 2048 10.1 -> 9.4, 2048 x 3072 (128 x 64 tiles before) 14.2 -> 12.0. Deeper
+// rings with one workgroup a CU (4 groups a stage, 6 or 8 slots), 8 wavefronts of 32 x 16 blocks and 128-byte rows were no
+// faster.
 template <int OUT>
 __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2))) void gemm_i8_few_kernel(
     const int8_t *__restrict__ X, const int8_t *__restrict__ W, const float *__restrict__ sxT,
@@ -1938,7 +1939,9 @@ void launch_gemm_bf16a(const uint16_t *X, const int8_t *B, const float *sx, cons
 // at the number resident) summed over the rounds + round x rounds + call. Fitted (us) to MI355X timings of the nine
 // configurations on 112 shapes (20 to 4000 rows over the LFM2 and SigLIP2 weights): within 5 % of a timing (rms), its pick
 // within 0.3 % of the fastest on average, where the W8A8 table above gave 3.7 % and up to 32 % (4000 x 4304 x 1152 97.6 ->
-// 73.8 us, 4000 x 1152 x 3456 58.0 -> 47.2, 1500 x 2048 x 2048 27.8 -> 25.5).
+// 73.8 us, 4000 x 1152 x 3456 58.0 -> 47.2, 1500 x 2048 x 2048 27.8 -> 25.5). On 144 other shapes its pick is 0.3 % from the
+// fastest on average, the table's 3.4 %; two are slower than with the table (800 x 1152 x 3456 16.7 -> 17.7, 600 x 1152 x 4352
+// 16.3 -> 17.2: 128 x 128 tiles in two K halves, which take longer the more CUs they fill).
 struct W8Cfg {
     int bm, bn, ksp, resident;
     double stage[4], round, call;
@@ -1990,10 +1993,12 @@ void launch_gemm_w8(const uint16_t *X, const int8_t *W, const float *sw, const u
     }
     // without that split, the tile and the split inside the workgroup by W8A16's own model
     const bool own = sk == 1 && !(knob_int(KNOB_GEMM_BM, 0) && knob_int(KNOB_GEMM_BN, 0));
-    const W8Cfg c = pick_w8(M, N, K);
+    int own_ksp = 1;
     if (own) {
+        const W8Cfg c = pick_w8(M, N, K);
         t.bm = c.bm;
         t.bn = c.bn;
+        own_ksp = c.ksp;
         tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     }
     const dim3 grid(tiles * sk);
@@ -2002,7 +2007,7 @@ void launch_gemm_w8(const uint16_t *X, const int8_t *W, const float *sw, const u
     // the others (LDS).
     // The LFM2Q_GEMM_KSPLIT knob (1 / 2 / 4) forces it (4 only for 64 x 64).
     const bool s64 = t.bm == 64 && t.bn == 64;
-    int ksp = own ? c.ksp : ((long)grid.x <= device_cus() && KT / sk >= 8) ? (s64 ? 4 : 2) : 1;
+    int ksp = own ? own_ksp : ((long)grid.x <= device_cus() && KT / sk >= 8) ? (s64 ? 4 : 2) : 1;
     if (const int f = knob_int(KNOB_GEMM_KSPLIT, 0)) ksp = f == 4 && s64 ? 4 : f == 2 ? 2 : 1;
     uint32_t *const w = static_cast<uint32_t *>(ws);
     if (sk > 1) {
