@@ -268,11 +268,6 @@ int lfm2q_quant_groups(const lfm2q_bf16 *x, int8_t *q, float *sT, int rows, int 
  * add_rmsnorm_q (L = H): if y != NULL, h = bf16(h + y) in place; x = bf16(w * bf16(h * rs)),
  *   rs = 1 / sqrt(sum(h^2) / H + eps). Replaces launch_add_rmsnorm_q kernels/int8_gemm.cu:590-642 (binding
  *   add_rmsnorm_q(), kernels/int8_gemm.cpp:122-132). */
-/* add_rmsnorm_q's h and x without the INT8 row: h = bf16(h + y) in place if y != NULL, x bf16 [rows, H] as above
- * (bit-identical). H % 8 == 0, H <= 8192, 16-byte aligned tensors. Replaces add_rmsnorm (kernels/lfm2_decode.cpp:33-38,
- * kernel kernels/lfm2_decode.cu:96-121). */
-int lfm2q_add_rmsnorm(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm2q_bf16 *w, lfm2q_bf16 *x, int rows, int H, float eps,
-                      lfm2q_stream_t stream);
 int lfm2q_add_rmsnorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm2q_bf16 *w, int8_t *q, float *s,
                         lfm2q_bf16 *x, int rows, int H, float eps, int grouped, lfm2q_stream_t stream);
 /* add_layernorm_q (L = D): if y != NULL, h = bf16(h + y) in place; x = bf16(((h - mean) * rstd) * w + b),
@@ -284,6 +279,11 @@ int lfm2q_add_layernorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm2q_bf16 *
  * Replaces launch_silu_mul_q kernels/int8_gemm.cu:646-682 (binding silu_mul_q(), kernels/int8_gemm.cpp:135-141). */
 int lfm2q_silu_mul_q(const lfm2q_bf16 *g, int8_t *q, float *s, lfm2q_bf16 *x, int rows, int I, int grouped,
                      lfm2q_stream_t stream);
+/* add_rmsnorm_q's h and x without the INT8 row: h = bf16(h + y) in place if y != NULL, x bf16 [rows, H] as there
+ * (bit-identical). H % 8 == 0, H <= 8192, 16-byte aligned tensors. Replaces add_rmsnorm (kernels/lfm2_decode.cpp:33-38,
+ * kernel kernels/lfm2_decode.cu:96-121). */
+int lfm2q_add_rmsnorm(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm2q_bf16 *w, lfm2q_bf16 *x, int rows, int H, float eps,
+                      lfm2q_stream_t stream);
 
 /* W8A8 GEMM with the dequant epilogue: Y[m, n] = bf16( g( ((float)acc[m, n] * sa[m]) * sb[n] + bias[n] ) ),
  * acc[m, n] = sum_k A[m, k] B[n, k] exact in int32, the three fp32 operations separately rounded (no FMA),

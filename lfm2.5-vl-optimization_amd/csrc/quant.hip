@@ -552,7 +552,7 @@ extern "C" int lfm2q_add_rmsnorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const lfm
     }
 #define LFM2Q_P(CH_)                                                                                                 \
     if (grouped)                                                                                                     \
-        add_rmsnorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, q, s, x, rows, H, eps);                    \
+        add_rmsnorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, q, s, x, rows, H, eps);                       \
     else                                                                                                             \
         add_rmsnorm_q_kernel<CH_, false><<<grid, 256, 0, st>>>(h, y, w, q, s, x, rows, H, eps)
     LFM2Q_CH_SWITCH(H, LFM2Q_P)
@@ -572,7 +572,7 @@ extern "C" int lfm2q_add_layernorm_q(lfm2q_bf16 *h, const lfm2q_bf16 *y, const l
     const hipStream_t st = (hipStream_t)stream;
 #define LFM2Q_P(CH_)                                                                                                 \
     if (grouped)                                                                                                     \
-        add_layernorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, b, q, s, x, rows, D, eps);             \
+        add_layernorm_q_kernel<CH_, true><<<grid, 256, 0, st>>>(h, y, w, b, q, s, x, rows, D, eps);                  \
     else                                                                                                             \
         add_layernorm_q_kernel<CH_, false><<<grid, 256, 0, st>>>(h, y, w, b, q, s, x, rows, D, eps)
     LFM2Q_CH_SWITCH(D, LFM2Q_P)
