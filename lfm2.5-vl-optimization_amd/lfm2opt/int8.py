@@ -139,9 +139,9 @@ class Int8Linear:
             rows = x2.shape[0]
             if not (self.a8 or quant_out):
                 y = self._gemm_w8a16(x2, gelu)
-                return y if len(lead) == 1 else y.view(*lead, self.N)
+                return y if lead == (rows,) else y.view(*lead, self.N)
             xq, sx = quantize_rows(x2, GROUP_COLS if quant_out else self.group)
         if quant_out:
             return self._gemm_int8_out(xq, sx, rows, gelu)
         y = self._gemm_bf16_out(xq, sx, rows, gelu)
-        return y if len(lead) == 1 else y.view(*lead, self.N)
+        return y if lead == (rows,) else y.view(*lead, self.N)

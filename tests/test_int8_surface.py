@@ -63,3 +63,22 @@ def test_int8_linear_construction(env):
         int8.Int8Linear()
     with pytest.raises(ValueError):
         int8.Int8Linear(q=q_ref)
+
+
+@pytest.mark.parametrize("a8", [False, True])
+def test_rows_wider_than_the_weight_are_refused(a8, monkeypatch):
+    """x [2, 2 K] holds whole rows of K, but no output [2, N] exists for it: an error, not four rows. (The kernels stand
+    still: the shapes are what is tested.)"""
+    from lfm2opt import int8
+
+    class Still:
+        def __getattr__(self, name):
+            return lambda *args: None
+
+    monkeypatch.setattr(int8, "int8_ext", Still)
+    layer = int8.Int8Linear(torch.randn(8, 64).to(torch.bfloat16), a8=a8)
+    assert layer(torch.zeros(2, 64, dtype=torch.bfloat16)).shape == (2, 8)
+    assert layer(torch.zeros(3, 2, 64, dtype=torch.bfloat16)).shape == (3, 2, 8)
+    assert layer(torch.zeros(64, dtype=torch.bfloat16)).shape == (8,)
+    with pytest.raises(RuntimeError, match="shape"):
+        layer(torch.zeros(2, 128, dtype=torch.bfloat16))
